@@ -249,7 +249,7 @@ __device__ void align_count_chunk(const IdT* __restrict__ ids, int R, int E, int
   for (int e = threadIdx.x; e < E + 1; e += NT) cc[(int64_t)c * (E + 1) + e] = cnt[e];
 }
 
-template <typename IdT, int NT, int QF>
+template <typename IdT, int NT, int QF, int U>
 __global__ __launch_bounds__(NT) void align_count_quant_kernel(const IdT* __restrict__ ids, int R, int E, int C,
                                                                int* __restrict__ cc, const uint4* __restrict__ x,
                                                                int64_t n_groups, int rule, void* q_codes,
@@ -258,11 +258,11 @@ __global__ __launch_bounds__(NT) void align_count_quant_kernel(const IdT* __rest
     align_count_chunk<IdT, NT>(ids, R, E, blockIdx.x, cc);
     return;
   }
-  const int64_t g = (int64_t)(blockIdx.x - C) * NT + threadIdx.x;
+  const int64_t wg = blockIdx.x - C;
   if (QF == 0)
-    dsv4::fp8_quant_group(x, g, g < n_groups, nullptr, (uint2*)q_codes, nullptr, (uint32_t*)q_scale);
+    dsv4::fp8_quant_wg<U, NT>(x, wg, n_groups, nullptr, (uint2*)q_codes, nullptr, (uint32_t*)q_scale);
   else if (QF == 1)
-    dsv4::mxfp4_quant_group(x, g, g < n_groups, rule, (uint32_t*)q_codes, (uint8_t*)q_scale, nullptr);
+    dsv4::mxfp4_quant_wg<U, NT>(x, wg, n_groups, rule, (uint32_t*)q_codes, (uint8_t*)q_scale, nullptr);
 }
 
 // Every chunk's workgroup sums the chunk counts itself (its exclusive
@@ -330,11 +330,11 @@ __global__ __launch_bounds__(NT) void moe_align_quant_kernel(const IdT* __restri
     align_body<IdT, NT>(ids, topk_w, R, K, E, block_m, max_blocks, o, n_shared);
     return;
   }
-  const int64_t g = (int64_t)(blockIdx.x - 1) * NT + threadIdx.x;
+  const int64_t wg = blockIdx.x - 1;
   if (QF == 0)
-    dsv4::fp8_quant_group(x, g, g < n_groups, nullptr, (uint2*)q_codes, nullptr, (uint32_t*)q_scale);
+    dsv4::fp8_quant_wg<1, NT>(x, wg, n_groups, nullptr, (uint2*)q_codes, nullptr, (uint32_t*)q_scale);
   else
-    dsv4::mxfp4_quant_group(x, g, g < n_groups, rule, (uint32_t*)q_codes, (uint8_t*)q_scale, nullptr);
+    dsv4::mxfp4_quant_wg<1, NT>(x, wg, n_groups, rule, (uint32_t*)q_codes, (uint8_t*)q_scale, nullptr);
 }
 
 // Decode-sized router + align in the layer's first launch (the router's top-k
@@ -355,11 +355,11 @@ __global__ __launch_bounds__(NT) void route_align_quant_kernel(RouteTopkArgs ra,
     align_body<int32_t, NT>(ra.out_ids, ra.out_w, ra.T * ra.K, ra.K, ra.E, block_m, max_blocks, o, n_shared);
     return;
   }
-  const int64_t g = (int64_t)(blockIdx.x - 1) * NT + threadIdx.x;
+  const int64_t wg = blockIdx.x - 1;
   if (QF == 0)
-    dsv4::fp8_quant_group(x, g, g < n_groups, nullptr, (uint2*)q_codes, nullptr, (uint32_t*)q_scale);
+    dsv4::fp8_quant_wg<1, NT>(x, wg, n_groups, nullptr, (uint2*)q_codes, nullptr, (uint32_t*)q_scale);
   else
-    dsv4::mxfp4_quant_group(x, g, g < n_groups, rule, (uint32_t*)q_codes, (uint8_t*)q_scale, nullptr);
+    dsv4::mxfp4_quant_wg<1, NT>(x, wg, n_groups, rule, (uint32_t*)q_codes, (uint8_t*)q_scale, nullptr);
 }
 
 }  // namespace
@@ -429,20 +429,23 @@ hipError_t launch_moe_align_chunked(const void* topk_ids, int ids_int64, const f
   int* cc = (int*)scratch;
   const int64_t n_groups = x ? n_elems / 8 : 0;
   constexpr int NT1 = 256;
-  const int64_t qwg = (n_groups + NT1 - 1) / NT1;
+  const int U = quant_groups_per_thread(n_groups);
+  const int64_t qwg = (n_groups + NT1 * U - 1) / (NT1 * U);
   if (C + qwg > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 g1((unsigned)(C + qwg));
   const size_t lds1 = sizeof(int) * (size_t)(E + 1);
-#define DSV4_CQ(IDT, QF)                                                                                    \
-  hipLaunchKernelGGL((align_count_quant_kernel<IDT, NT1, QF>), g1, dim3(NT1), lds1, st, (const IDT*)topk_ids, \
+#define DSV4_CQU(IDT, QF, U_)                                                                                    \
+  hipLaunchKernelGGL((align_count_quant_kernel<IDT, NT1, QF, U_>), g1, dim3(NT1), lds1, st, (const IDT*)topk_ids, \
                      R, E, C, cc, (const uint4*)x, n_groups, rule, q_codes, q_scale)
+#define DSV4_CQ(IDT, QF) if (U == 2) DSV4_CQU(IDT, QF, 2); else DSV4_CQU(IDT, QF, 1)
   const int qf = x ? qfmt : 2;  // 2: count only
   if (ids_int64) {
-    if (qf == 0) DSV4_CQ(long long, 0); else if (qf == 1) DSV4_CQ(long long, 1); else DSV4_CQ(long long, 2);
+    if (qf == 0) { DSV4_CQ(long long, 0); } else if (qf == 1) { DSV4_CQ(long long, 1); } else { DSV4_CQ(long long, 2); }
   } else {
-    if (qf == 0) DSV4_CQ(int32_t, 0); else if (qf == 1) DSV4_CQ(int32_t, 1); else DSV4_CQ(int32_t, 2);
+    if (qf == 0) { DSV4_CQ(int32_t, 0); } else if (qf == 1) { DSV4_CQ(int32_t, 1); } else { DSV4_CQ(int32_t, 2); }
   }
 #undef DSV4_CQ
+#undef DSV4_CQU
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   // the layout needs one thread per expert: 256 threads up to 256 experts, 1024 above

@@ -45,35 +45,6 @@ DSV4_DEV int ceil_log2(float v) {
 // E8M0 byte -> fp32 scale (npu_ops.py:35-44).
 DSV4_DEV float e8m0_to_f32(uint32_t b) { return pow2f((int)b - 127); }
 
-// |v| (already divided by the block scale, |v| <= 448) -> E4M3fn magnitude code
-// with round-to-nearest-even. The binade exponent is clamped at -6 so that the
-// subnormal range uses the same formula; a carry out of the mantissa moves into
-// the exponent field by the addition itself.
-DSV4_DEV uint32_t e4m3_mag_code(float a) {
-  int E = (a < 0.015625f) ? -6 : floor_log2(a);
-  float r = __builtin_rintf(a * pow2f(3 - E));
-  int code = ((E + 7) << 3) + (int)r - 8;
-  return (a == 0.0f) ? 0u : (uint32_t)code;
-}
-DSV4_DEV float e4m3_mag_value(uint32_t c) {
-  uint32_t e = (c >> 3) & 15u, m = c & 7u;
-  return (e == 0) ? (float)m * 0.001953125f : pow2f((int)e - 7) * (1.0f + 0.125f * (float)m);
-}
-
-// |v| in [0, 6] -> E2M1 magnitude index 0..7 (round-to-nearest-even on the
-// E2M1 grid; equal to the reference's searchsorted/tie-to-even rule,
-// npu_ops.py:53-67).
-DSV4_DEV uint32_t e2m1_mag_code(float a) {
-  int E = (a < 1.0f) ? 0 : floor_log2(a);
-  float r = __builtin_rintf(a * pow2f(1 - E));
-  int code = ((E + 1) << 1) + (int)r - 2;
-  return (a == 0.0f) ? 0u : (uint32_t)code;
-}
-DSV4_DEV float e2m1_mag_value(uint32_t c) {
-  // 0, .5, 1, 1.5, 2, 3, 4, 6
-  return (c < 2) ? 0.5f * (float)c : pow2f((int)(c >> 1) - 1) * (1.0f + 0.5f * (float)(c & 1));
-}
-
 // Wave helpers (wave64).
 DSV4_DEV float wave_max_xor(float v, int width) {
   for (int o = width >> 1; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));

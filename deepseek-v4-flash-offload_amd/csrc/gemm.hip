@@ -361,17 +361,18 @@ DSV4_DEV void quantise_h_mxfp4(const Dsv4GemmArgs& p, const uint32_t (*hb)[2], c
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float v0 = dsv4::bf16_to_f32(hb[i][0]), v1 = dsv4::bf16_to_f32(hb[i][1]);
-    const float amax = dsv4::wave_max_xor(fmaxf(fabsf(v0), fabsf(v1)), 16);
+    const float amax = dsv4::row16_max(fmaxf(fabsf(v0), fabsf(v1)));
     const int k = dsv4::mxfp4_block_exp(amax, p.hq_rule);
     const float inv = dsv4::pow2f(-k);
-    const uint32_t n0 = dsv4::mxfp4_nibble(v0, inv, p.hq_rule), n1 = dsv4::mxfp4_nibble(v1, inv, p.hq_rule);
-    const uint32_t o0 = (uint32_t)__shfl_xor((int)n0, 1, 64), o1 = (uint32_t)__shfl_xor((int)n1, 1, 64);
+    const float y0 = dsv4::mxfp4_clamped(v0, inv, p.hq_rule), y1 = dsv4::mxfp4_clamped(v1, inv, p.hq_rule);
+    const uint32_t own = dsv4::e2m1_pair<0>(0u, y0, y1);  // low nibble: tile 0, high: tile 1
+    const uint32_t nbr = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own, 0xb1, 0xf, 0xf, false);  // lane ^ 1
     const int f = fr[i];
     if (f < p.R) {
       uint8_t* row = p.hq_codes + (int64_t)f * (p.N / 2) + col0 / 2;
       if ((r16 & 1) == 0) {  // low nibble = even column
-        row[r16 / 2] = (uint8_t)(n0 | (o0 << 4));
-        row[8 + r16 / 2] = (uint8_t)(n1 | (o1 << 4));
+        row[r16 / 2] = (uint8_t)((own & 0xfu) | (nbr << 4));
+        row[8 + r16 / 2] = (uint8_t)((own >> 4) & 0xfu) | (uint8_t)(nbr & 0xf0u);
       }
       if (r16 == 0) p.hq_scale[(int64_t)f * (p.N / 32) + col0 / 32] = (uint8_t)(k + 127);
     }
@@ -897,8 +898,8 @@ __attribute__((always_inline)) DSV4_DEV void tiled_block(const Dsv4GemmArgs& p,
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float m = dsv4::wave_max_xor(
-              fmaxf(fabsf(dsv4::bf16_to_f32(hb[mt][i][0])), fabsf(dsv4::bf16_to_f32(hb[mt][i][1]))), 16);
+          const float m = dsv4::row16_max(
+              fmaxf(fabsf(dsv4::bf16_to_f32(hb[mt][i][0])), fabsf(dsv4::bf16_to_f32(hb[mt][i][1]))));
           if (r16 == 0) am[wave * BM + 16 * mt + 4 * g + i] = m;
         }
       __syncthreads();

@@ -156,22 +156,25 @@ __global__ __launch_bounds__(256) void mxfp4_dequant_multi_kernel(Dsv4DequantJob
 }
 
 // ---------------------------------------------------------------------------
-// Activation quantisers (bodies in quant_dev.h): one thread per 8-element group.
+// Activation quantisers (bodies in quant_dev.h): U 8-element groups per thread. Bound
+// by HBM at the sizes of a prompt chunk and by the launch below ~1000 rows. [4096, 4096]
+// bf16: FP8 21.6 us -> 11.5 us (4.4 TB/s), MXFP4 20.6 -> 8.6 us (4.9 TB/s) against the
+// former integer rounding, whose ~30 VALU instructions per element bound the kernels.
 // ---------------------------------------------------------------------------
+template <int U>
 __global__ __launch_bounds__(256) void fp8_act_quant_kernel(const uint4* __restrict__ x, int64_t n_groups,
                                                              uint4* __restrict__ rt, uint2* __restrict__ codes,
                                                              float* __restrict__ scale_f32,
                                                              uint32_t* __restrict__ scale_e8m0x4) {
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  fp8_quant_group(x, g, g < n_groups, rt, codes, scale_f32, scale_e8m0x4);  // n_groups % 16 == 0
+  fp8_quant_wg<U, 256>(x, blockIdx.x, n_groups, rt, codes, scale_f32, scale_e8m0x4);
 }
 
+template <int U>
 __global__ __launch_bounds__(256) void mxfp4_act_quant_kernel(const uint4* __restrict__ x, int64_t n_groups,
                                                                int rule, uint32_t* __restrict__ packed,
                                                                uint8_t* __restrict__ scale,
                                                                uint4* __restrict__ dq) {
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  mxfp4_quant_group(x, g, g < n_groups, rule, packed, scale, dq);  // n_groups % 4 == 0
+  mxfp4_quant_wg<U, 256>(x, blockIdx.x, n_groups, rule, packed, scale, dq);
 }
 
 // ---------------------------------------------------------------------------
@@ -356,20 +359,30 @@ hipError_t launch_mxfp4_dequant_multi(const Dsv4DequantJobs& jobs, hipStream_t s
 
 hipError_t launch_fp8_act_quant(const uint16_t* x, int64_t n_elems, uint16_t* rt, uint8_t* codes,
                                 float* scale_f32, uint8_t* scale_e8m0x4, hipStream_t st) {
-  int64_t n_groups = n_elems / 8;
+  const int64_t n_groups = n_elems / 8;
   if (n_groups == 0) return hipSuccess;
-  int grid = (int)((n_groups + 255) / 256);
-  hipLaunchKernelGGL(fp8_act_quant_kernel, dim3(grid), dim3(256), 0, st, (const uint4*)x, n_groups,
-                     (uint4*)rt, (uint2*)codes, scale_f32, (uint32_t*)scale_e8m0x4);
+  const int U = quant_groups_per_thread(n_groups);
+  const int64_t grid = (n_groups + 256 * U - 1) / (256 * U);
+  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+#define DSV4_FQ(U_)                                                                                               \
+  hipLaunchKernelGGL((fp8_act_quant_kernel<U_>), dim3((unsigned)grid), dim3(256), 0, st, (const uint4*)x, n_groups, \
+                     (uint4*)rt, (uint2*)codes, scale_f32, (uint32_t*)scale_e8m0x4)
+  if (U == 2) DSV4_FQ(2); else DSV4_FQ(1);
+#undef DSV4_FQ
   return hipGetLastError();
 }
 
 hipError_t launch_mxfp4_act_quant(const uint16_t* x, int64_t n_elems, int rule, uint8_t* packed,
                                   uint8_t* scale, uint16_t* dq, hipStream_t st) {
-  int64_t n_groups = n_elems / 8;
+  const int64_t n_groups = n_elems / 8;
   if (n_groups == 0) return hipSuccess;
-  int grid = (int)((n_groups + 255) / 256);
-  hipLaunchKernelGGL(mxfp4_act_quant_kernel, dim3(grid), dim3(256), 0, st, (const uint4*)x, n_groups,
-                     rule, (uint32_t*)packed, scale, (uint4*)dq);
+  const int U = quant_groups_per_thread(n_groups);
+  const int64_t grid = (n_groups + 256 * U - 1) / (256 * U);
+  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+#define DSV4_MQ(U_)                                                                                                 \
+  hipLaunchKernelGGL((mxfp4_act_quant_kernel<U_>), dim3((unsigned)grid), dim3(256), 0, st, (const uint4*)x, n_groups, \
+                     rule, (uint32_t*)packed, scale, (uint4*)dq)
+  if (U == 2) DSV4_MQ(2); else DSV4_MQ(1);
+#undef DSV4_MQ
   return hipGetLastError();
 }

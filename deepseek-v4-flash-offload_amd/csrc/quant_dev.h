@@ -3,7 +3,7 @@
 // One thread owns 8 consecutive bf16 elements (group g); the lanes of one
 // quantisation block are consecutive lanes of one wave (16 lanes per 128-element
 // FP8 block, 4 lanes per 32-element MXFP4 block), so the block's amax is a
-// wave-local xor reduction. The caller maps lanes to groups so that g % 16
+// reduction over one DPP row (quad). The caller maps lanes to groups so that g % 16
 // (resp. g % 4) equals the lane's position in its block.
 #pragma once
 #include "common.h"
@@ -20,20 +20,34 @@ DSV4_DEV int fp8_block_exp(float amax) {
   return ceil_log2(vs);
 }
 
-// E4M3fn code of element f of a block with inverse scale inv = 2^-k
+// Largest value over the 16 lanes of a DPP row (the lanes of one FP8 block), in all of
+// them; quad_max: over 4 consecutive lanes (one MXFP4 block). Lane permutes inside the
+// VALU: a shuffle through the LDS crossbar per step was the longest chain of a quantiser.
+template <int CTRL>
+DSV4_DEV float dpp_max(float v) {
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false)));
+}
+DSV4_DEV float quad_max(float v) { return dpp_max<0x4e>(dpp_max<0xb1>(v)); }  // quad_perm xor 1, xor 2
+DSV4_DEV float row16_max(float v) { return dpp_max<0x140>(dpp_max<0x141>(quad_max(v))); }  // half-row, row mirror
+
+// E4M3fn codes of f[0..3] times inv = 2^-k, byte 0 first: the clamp of act_quant, then
+// the hardware converter, which rounds to nearest even as torch's cast does (the same
+// code as the former integer rounding for every fp32 in +-448; the clamp maps NaN to -448).
+DSV4_DEV uint32_t fp8_codes4(const float* f, float inv) {
+  float y[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = fminf(fmaxf(f[i] * inv, -448.0f), 448.0f);
+  const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], lo, true);
+}
 DSV4_DEV uint32_t fp8_code(float f, float inv) {
-  float y = fminf(fmaxf(f * inv, -448.0f), 448.0f);
-  uint32_t neg = __float_as_uint(y) >> 31;
-  return e4m3_mag_code(fabsf(y)) | (neg << 7);
+  const float y = fminf(fmaxf(f * inv, -448.0f), 448.0f);
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y, y, 0, false) & 0xffu;
 }
 
-// `live` must be the same for the 16 lanes of a block.
-DSV4_DEV void fp8_quant_group(const uint4* __restrict__ x, int64_t g, bool live, uint4* __restrict__ rt,
-                              uint2* __restrict__ codes, float* __restrict__ scale_f32,
-                              uint32_t* __restrict__ scale_e8m0x4) {
-  uint4 v = live ? x[g] : make_uint4(0, 0, 0, 0);
-  uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  float f[8];
+// 8 bf16 of one 16-byte load as floats; returns their largest magnitude
+DSV4_DEV float unpack8(const uint4 v, float* f) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -41,28 +55,52 @@ DSV4_DEV void fp8_quant_group(const uint4* __restrict__ x, int64_t g, bool live,
     f[2 * i + 1] = bf16_to_f32(w[i] >> 16);
     amax = fmaxf(amax, fmaxf(fabsf(f[2 * i]), fabsf(f[2 * i + 1])));
   }
-  amax = wave_max_xor(amax, 16);
+  return amax;
+}
+
+// Group g (already loaded: v) of a tensor; `live` must be the same for the 16 lanes of a block.
+DSV4_DEV void fp8_quant_loaded(const uint4 v, int64_t g, bool live, uint4* __restrict__ rt, uint2* __restrict__ codes,
+                               float* __restrict__ scale_f32, uint32_t* __restrict__ scale_e8m0x4) {
+  float f[8];
+  const float amax = row16_max(unpack8(v, f));
   const int k = fp8_block_exp(amax);
-  float s = pow2f(k), inv = pow2f(-k);
-  uint32_t c[8];
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    c[i] = fp8_code(f[i], inv);
-    const uint32_t neg = c[i] >> 7, mag = c[i] & 0x7fu;
-    float q = e4m3_mag_value(mag) * s;
-    uint32_t b = f32_to_bf16(neg ? -q : q);
-    if (i & 1) o[i >> 1] |= b << 16; else o[i >> 1] = b;
-  }
+  const float inv = pow2f(-k);
+  const uint2 c = make_uint2(fp8_codes4(f, inv), fp8_codes4(f + 4, inv));
   if (!live) return;
-  if (rt) rt[g] = make_uint4(o[0], o[1], o[2], o[3]);
-  if (codes) codes[g] = make_uint2(c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24),
-                                   c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24));
+  if (rt) {  // code * 2^k has at most 4 significant bits, so the upper half of the fp32 is the bf16
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    const float s = pow2f(k);
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int w = (int)(i < 2 ? c.x : c.y);
+      const f32x2 q = (i & 1) ? __builtin_amdgcn_cvt_pk_f32_fp8(w, true) : __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
+      o[i] = (__float_as_uint(q.x * s) >> 16) | (__float_as_uint(q.y * s) & 0xffff0000u);
+    }
+    rt[g] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+  if (codes) codes[g] = c;
   if ((g & 15) == 0) {
     const int64_t blk = g >> 4;
-    if (scale_f32) scale_f32[blk] = s;
+    if (scale_f32) scale_f32[blk] = pow2f(k);
     if (scale_e8m0x4) scale_e8m0x4[blk] = (uint32_t)(k + 127) * 0x01010101u;
   }
+}
+
+// A workgroup's share of a tensor: U groups per thread, NT apart (consecutive lanes on
+// consecutive groups), from group `wg` * U * NT on; every load is issued before the first
+// is used. n_groups is a multiple of 16, so a block's lanes are live together.
+template <int U, int NT>
+DSV4_DEV void fp8_quant_wg(const uint4* __restrict__ x, int64_t wg, int64_t n_groups, uint4* __restrict__ rt,
+                           uint2* __restrict__ codes, float* __restrict__ scale_f32,
+                           uint32_t* __restrict__ scale_e8m0x4) {
+  const int64_t g0 = wg * (U * NT) + threadIdx.x;
+  uint4 v[U];
+#pragma unroll
+  for (int i = 0; i < U; ++i) v[i] = g0 + i * NT < n_groups ? x[g0 + i * NT] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < U; ++i)
+    fp8_quant_loaded(v[i], g0 + i * NT, g0 + i * NT < n_groups, rt, codes, scale_f32, scale_e8m0x4);
 }
 
 // MXFP4 activation quant, per 32 elements.
@@ -83,54 +121,61 @@ DSV4_DEV int mxfp4_block_exp(float amax, int rule) {
   return (amax == 0.0f) ? -127 : min(max(floor_log2(amax) - 2, -127), 127);
 }
 
-// sign-magnitude E2M1 nibble of element f of a block with inverse scale inv = 2^-k
-DSV4_DEV uint32_t mxfp4_nibble(float f, float inv, int rule) {
-  float y = f * inv;
-  uint32_t neg;
-  float a;
-  if (rule == 0) {
-    y = fminf(fmaxf(y, -6.0f), 6.0f);
-    neg = (y < 0.0f) ? 1u : 0u;
-    a = fabsf(y);
-  } else {
-    neg = __float_as_uint(f) >> 31;
-    a = fminf(fabsf(y), 6.0f);
-  }
-  return e2m1_mag_code(a) | (neg << 3);
+// Two floats already in [-6, 6] as sign-magnitude E2M1 nibbles in byte SEL of `old` (low
+// nibble = a): the hardware converter (round to nearest even, the sign of the input).
+template <int SEL>
+DSV4_DEV uint32_t e2m1_pair(uint32_t old, float a, float b) {
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(old, a, b, 1.0f, SEL);
 }
 
-// `live` must be the same for the 4 lanes of a block.
-DSV4_DEV void mxfp4_quant_group(const uint4* __restrict__ x, int64_t g, bool live, int rule,
-                                uint32_t* __restrict__ packed, uint8_t* __restrict__ scale,
-                                uint4* __restrict__ dq) {
-  uint4 v = live ? x[g] : make_uint4(0, 0, 0, 0);
-  uint32_t w[4] = {v.x, v.y, v.z, v.w};
+// Element f times inv = 2^-k clamped to the E2M1 range, with the sign its nibble takes:
+// rule 0 the sign of the clamped quotient (NaN clamps to -6), +0 for either zero; rule 1
+// the sign bit of f.
+DSV4_DEV float mxfp4_clamped(float f, float inv, int rule) {
+  if (rule == 0) return fminf(fmaxf(f * inv, -6.0f), 6.0f) + 0.0f;  // -0 + 0 = +0
+  return copysignf(fminf(fabsf(f * inv), 6.0f), f);
+}
+
+// Group g (already loaded: v) of a tensor; `live` must be the same for the 4 lanes of a block.
+DSV4_DEV void mxfp4_quant_loaded(const uint4 v, int64_t g, bool live, int rule, uint32_t* __restrict__ packed,
+                                 uint8_t* __restrict__ scale, uint4* __restrict__ dq) {
   float f[8];
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = bf16_to_f32(w[i] & 0xffffu);
-    f[2 * i + 1] = bf16_to_f32(w[i] >> 16);
-    amax = fmaxf(amax, fmaxf(fabsf(f[2 * i]), fabsf(f[2 * i + 1])));
-  }
-  amax = wave_max_xor(amax, 4);
+  const float amax = quad_max(unpack8(v, f));
   const int k = mxfp4_block_exp(amax, rule);
-  float s = pow2f(k), inv = pow2f(-k);
-  uint32_t pk = 0;
-  uint32_t o[4];
+  const float inv = pow2f(-k);
+  if (rule == 0) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t nib = mxfp4_nibble(f[i], inv, rule);
-    pk |= nib << (4 * i);
-    const uint32_t neg = nib >> 3, mag = nib & 7u;
-    float q = e2m1_mag_value(mag) * s;
-    uint32_t b = f32_to_bf16(neg ? -q : q);
-    if (i & 1) o[i >> 1] |= b << 16; else o[i >> 1] = b;
+    for (int i = 0; i < 8; ++i) f[i] = mxfp4_clamped(f[i], inv, 0);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = mxfp4_clamped(f[i], inv, 1);
   }
+  uint32_t pk = e2m1_pair<0>(0u, f[0], f[1]);
+  pk = e2m1_pair<1>(pk, f[2], f[3]);
+  pk = e2m1_pair<2>(pk, f[4], f[5]);
+  pk = e2m1_pair<3>(pk, f[6], f[7]);
   if (!live) return;
   packed[g] = pk;
-  if (dq) dq[g] = make_uint4(o[0], o[1], o[2], o[3]);
+  if (dq) {  // nibble * 2^k, exact in bf16 (two significant bits; sign of zero kept)
+    const float s = pow2f(k);
+    dq[g] = make_uint4(__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pk, s, 0)),
+                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pk, s, 1)),
+                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pk, s, 2)),
+                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pk, s, 3)));
+  }
   if ((g & 3) == 0) scale[g >> 2] = (uint8_t)(k + 127);
+}
+
+// As fp8_quant_wg (n_groups a multiple of 4).
+template <int U, int NT>
+DSV4_DEV void mxfp4_quant_wg(const uint4* __restrict__ x, int64_t wg, int64_t n_groups, int rule,
+                             uint32_t* __restrict__ packed, uint8_t* __restrict__ scale, uint4* __restrict__ dq) {
+  const int64_t g0 = wg * (U * NT) + threadIdx.x;
+  uint4 v[U];
+#pragma unroll
+  for (int i = 0; i < U; ++i) v[i] = g0 + i * NT < n_groups ? x[g0 + i * NT] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < U; ++i) mxfp4_quant_loaded(v[i], g0 + i * NT, g0 + i * NT < n_groups, rule, packed, scale, dq);
 }
 
 }  // namespace dsv4

@@ -181,3 +181,25 @@ def test_mxfp4_gemv_rejects_bad_shapes(gpu):
     with pytest.raises(ops._lib.Dsv4Error, match="at most 16"):
         ops.mxfp4_gemv(torch.zeros(17, 64, dtype=torch.bfloat16, device=gpu),
                        torch.zeros(8, 32, dtype=torch.uint8, device=gpu), torch.zeros(8, 2, dtype=torch.uint8, device=gpu))
+
+
+@pytest.mark.parametrize("rows", [4095, 4096, 4099])   # one group per thread, two, two with a partial workgroup
+def test_act_quant_rows_do_not_depend_on_the_launch(gpu, rows):
+    """Row blocks are independent, so a large tensor's codes equal those of its parts (the small
+    launch, which the tests above compare with the oracle), non-finite values included."""
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    x = torch.randn(rows, 4096, generator=g, device=gpu).to(torch.bfloat16)
+    x[rows - 1, :6] = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0, 1e-30, -1e-30], device=gpu)
+    rt, dq = torch.empty_like(x), torch.empty_like(x)
+    whole = ops.fp8_act_quant(x, 128, rt=rt, want_codes=True, want_scale=True, want_e8m0x4=True)
+    packed, scale, _ = ops.mxfp4_act_quant(x, RULE_OCP_FLOOR, dq=dq)
+    for a, b in ((0, 1000), (rows - 1000, rows)):
+        part = x[a:b].contiguous()
+        prt, pdq = torch.empty_like(part), torch.empty_like(part)
+        want = ops.fp8_act_quant(part, 128, rt=prt, want_codes=True, want_scale=True, want_e8m0x4=True)
+        for k in ("codes", "scale", "e8m0x4"):
+            assert torch.equal(whole[k][a:b], want[k]), k
+        assert torch.equal(rt[a:b].view(torch.int16), prt.view(torch.int16))
+        p, s, _ = ops.mxfp4_act_quant(part, RULE_OCP_FLOOR, dq=pdq)
+        assert torch.equal(packed[a:b], p) and torch.equal(scale[a:b], s)
+        assert torch.equal(dq[a:b].view(torch.int16), pdq.view(torch.int16))
