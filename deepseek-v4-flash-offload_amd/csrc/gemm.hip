@@ -334,13 +334,9 @@ DSV4_DEV void store_tile(const Dsv4GemmArgs& p, const v4f* acc, int row0, int co
       const float w = (!SH || f < p.R - p.shared_a_rows) ? p.topk_w[f] : 1.0f;
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        float gt = dsv4::bf16_to_f32(dsv4::f32_to_bf16(acc[t][i]));
-        float up = dsv4::bf16_to_f32(dsv4::f32_to_bf16(acc[t + 2][i]));
-        if (p.swiglu_limit > 0.0f) {
-          up = fminf(fmaxf(up, -p.swiglu_limit), p.swiglu_limit);
-          gt = fminf(gt, p.swiglu_limit);
-        }
-        const float h = gt / (1.0f + expf(-gt)) * up * w;
+        const float gt = dsv4::bf16_to_f32(dsv4::f32_to_bf16(acc[t][i]));
+        const float up = dsv4::bf16_to_f32(dsv4::f32_to_bf16(acc[t + 2][i]));
+        const float h = dsv4::swiglu(gt, up, w, p.swiglu_limit);
         const uint32_t b = dsv4::f32_to_bf16(h);
         if (hb) hb[i][t] = b;
         if (!p.hq_skip_h) orow[16 * t] = (uint16_t)b;

@@ -83,6 +83,7 @@ struct Cfg {
   static constexpr int TT = BM / WM / 32;      // 32-row token tiles per wave
   static constexpr int WT = kBN / WN / 32;     // 32-row weight tiles per wave
   static constexpr int WGS = HALF ? 2 : 1;     // workgroups per CU
+  static constexpr int LDS_EPI = 72 * 1024;    // LDS the epilogue may use (the ring's, checked below)
 };
 
 template <int AFMT, bool HALF>
@@ -108,6 +109,7 @@ struct Big {
   static constexpr int SV = SCL / (kNT * 16);         // scale loads per thread per super-stage
   static constexpr int LDS = NB * STAGE + 2 * SCL;
   static_assert(LDS * Cfg<AFMT, HALF>::WGS <= 160 * 1024, "the stage ring and two scale super-stages must fit the LDS");
+  static_assert(LDS >= Cfg<AFMT, HALF>::LDS_EPI, "the epilogue's share");
   static_assert(BCH == 8 && (ACH * 1024) == kBM * (AFMT == 0 ? kKS : kKS / 2), "chunking");
   static_assert(AV * G::NW == ACH && BV * G::NW == BCH && SV * kNT * 16 == SCL, "loads per thread");
   static_assert(L * NB + SV < 64, "vmcnt holds 6 bits");
@@ -313,17 +315,6 @@ DSV4_DEV uint32_t pk_bf16(float a, float b) {
 DSV4_DEV float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 DSV4_DEV float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// silu(min(g, L)) * clamp(u, +-L) * w for bf16-rounded g, u, with silu(g) = g / (1 + e^-g)
-// written exactly as the 16/64-row kernels' epilogue (expf, IEEE divide), so a token row
-// gets the same h whichever kernel its expert runs on (deepseek_v4.py:184-187)
-DSV4_DEV float big_swiglu(float gt, float up, float w, float limit) {
-  if (limit > 0.0f) {
-    up = fminf(fmaxf(up, -limit), limit);
-    gt = fminf(gt, limit);
-  }
-  return gt / (1.0f + expf(-gt)) * up * w;
-}
-
 // 4 E4M3 codes of a * inv .. d * inv (inv = 2^-k), byte 0 = a
 DSV4_DEV uint32_t pk_fp8x4(float a, float b, float c, float d, float inv) {
   const float m = 448.0f;
@@ -364,6 +355,45 @@ DSV4_DEV void big_tile_of_block(int& mb, int& nt) {
   nt = 8 * (gi % ngroups) + (w & 7);
 }
 
+// Staged stores. A lane holds 4-column runs of one row, so storing from the accumulators
+// writes 8 bytes (bf16), 4 (E4M3) or 2 (E2M1) per lane to 32 rows per instruction: the
+// 1 GB of down outputs of a 16384-token layer took 390 us of the kernel's 1240 that way
+// (bf16 profile; 380 of 1044 a4w4). Each wave instead puts a token tile's rows into its
+// own part of the LDS (the ring is free by then) and stores them in whole 16-byte pieces,
+// consecutive lanes on consecutive pieces of a row. Only the wave's own lanes exchange
+// data, and a wave's LDS accesses complete in order, so no barrier is needed.
+constexpr int kStageOff = 4096;  // bytes at the start of the LDS left to the FP8 row maxima
+template <int ROWB>
+constexpr int stage_pitch() { return ROWB + 16; }
+
+DSV4_DEV void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Stores 32 * NTT staged rows of ROWB bytes (NTT token tiles whose lane r32 holds flat
+// index fr[tile]) to base + f * row_stride; rows with f >= R (padding) are left out.
+template <int ROWB, int NTT>
+DSV4_DEV void store_staged_rows(const uint8_t* st, int lane, const int* fr, int R, uint8_t* base, int64_t row_stride) {
+  constexpr int CPR = ROWB / 16;        // 16-byte pieces per row
+  constexpr int RPI = 64 / CPR;         // rows per store instruction
+  constexpr int IT = 32 * NTT / RPI;
+  static_assert(CPR * RPI == 64 && IT * RPI == 32 * NTT, "whole store instructions");
+  wave_lds_fence();
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int row = it * RPI + lane / CPR, ch = lane % CPR;
+    const int t0 = it * RPI / 32;
+    int f;
+    if constexpr (RPI == 64) f = lane < 32 ? fr[t0] : fr[t0 + 1];
+    else f = __shfl(fr[t0], row & 31, 64);
+    const v4i v = *(const v4i*)(st + row * stage_pitch<ROWB>() + 16 * ch);
+    if (f < R) *(v4i*)(base + (int64_t)f * row_stride + 16 * ch) = v;
+  }
+  wave_lds_fence();
+}
+
 // Epilogue of a large-tile workgroup (every wave is past the operand ring, so the LDS is
 // free): gate/up - SwiGLU x routing weight, bf16 h and/or its quantisation (hq_mode);
 // down - bf16 outputs. acc[tt][wt]: register r of lane l = weight column 8(r/4) + 4(l/32) +
@@ -371,8 +401,15 @@ DSV4_DEV void big_tile_of_block(int& mb, int& nt) {
 // (BM rows, WM x WN waves of TT x WT tiles).
 template <class G, bool GATEUP>
 DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uint8_t* lds, int c0, int wm, int wn,
-                           int r32, int g2, const int* fr, const float* wr) {
+                           int lane, const int* fr, const float* wr) {
   constexpr int kBM = G::BM, H = G::WT / 2;
+  typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+  const int r32 = lane & 31, g2 = lane >> 5;
+  constexpr int kStageRow = GATEUP ? 64 * H : 64 * G::WT;  // bytes of the widest staged row (bf16)
+  constexpr int kStage = 32 * stage_pitch<kStageRow>();    // per wave
+  static_assert(kStageOff + G::NW * kStage <= G::LDS_EPI, "the staged rows fit the operand ring");
+  static_assert(G::WN * kBM * 4 <= kStageOff, "the row maxima stay clear of them");
+  uint8_t* st = lds + kStageOff + (wm * G::WN + wn) * kStage;
   if (GATEUP) {
     const int cw = c0 + 32 * H * wn;  // this wave's first of 32 H intermediate columns
     // h for columns cw + 32 h + 8 q + 4 g2 + e of token tile tt, packed bf16 pairs
@@ -391,8 +428,8 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
             // gate (tile h) and up (tile H + h) of the same column, rounded to bf16
             const uint32_t gu0 = pk_bf16(acc[tt][h][r], acc[tt][H + h][r]);
             const uint32_t gu1 = pk_bf16(acc[tt][h][r + 1], acc[tt][H + h][r + 1]);
-            const uint32_t hw = pk_bf16(big_swiglu(bf16_lo(gu0), bf16_hi(gu0), wr[tt], p.swiglu_limit),
-                                        big_swiglu(bf16_lo(gu1), bf16_hi(gu1), wr[tt], p.swiglu_limit));
+            const uint32_t hw = pk_bf16(dsv4::swiglu(bf16_lo(gu0), bf16_hi(gu0), wr[tt], p.swiglu_limit),
+                                        dsv4::swiglu(bf16_lo(gu1), bf16_hi(gu1), wr[tt], p.swiglu_limit));
             hp[tt][h][q][e >> 1] = hw;
             m = fmaxf(m, fmaxf(fabsf(bf16_lo(hw)), fabsf(bf16_hi(hw))));
           }
@@ -400,36 +437,39 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
       }
     if (!p.hq_skip_h && p.out) {
 #pragma unroll
-      for (int tt = 0; tt < G::TT; ++tt)
-        if (fr[tt] < p.R)
+      for (int tt = 0; tt < G::TT; ++tt) {
 #pragma unroll
-          for (int h = 0; h < H; ++h)
+        for (int h = 0; h < H; ++h)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-              *(v2u*)(p.out + (int64_t)fr[tt] * p.N + cw + 32 * h + 8 * q + 4 * g2) =
-                  v2u{hp[tt][h][q][0], hp[tt][h][q][1]};
-            }
+          for (int q = 0; q < 4; ++q)
+            *(v2u*)(st + r32 * stage_pitch<64 * H>() + 64 * h + 16 * q + 8 * g2) =
+                v2u{hp[tt][h][q][0], hp[tt][h][q][1]};
+        store_staged_rows<64 * H, 1>(st, lane, fr + tt, p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
+      }
     }
     if (p.hq_mode == 2) {  // MXFP4 h: one 32-column block per (tt, h), half of it in each lane of a pair
+      constexpr int NS = H == 1 ? 2 : 1;  // token tiles per staged batch (16 H bytes per row)
+      static_assert(G::TT % NS == 0, "whole batches");
 #pragma unroll
-      for (int tt = 0; tt < G::TT; ++tt)
+      for (int tb = 0; tb < G::TT; tb += NS) {
 #pragma unroll
-        for (int h = 0; h < H; ++h) {
-          const int k = dsv4::mxfp4_block_exp(max_pair(rmax[tt][h]), p.hq_rule);
-          const float inv = dsv4::pow2f(-k);
-          if (fr[tt] < p.R) {
-            const int col = cw + 32 * h;
+        for (int ts = 0; ts < NS; ++ts)
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            const int tt = tb + ts;
+            const int k = dsv4::mxfp4_block_exp(max_pair(rmax[tt][h]), p.hq_rule);
+            const float inv = dsv4::pow2f(-k);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
               const uint32_t nib = pk_fp4x2(bf16_lo(w0), bf16_hi(w0), inv, p.hq_rule) |
                                    pk_fp4x2(bf16_lo(w1), bf16_hi(w1), inv, p.hq_rule) << 8;
-              *(uint16_t*)(p.hq_codes + (int64_t)fr[tt] * (p.N / 2) + (col + 8 * q + 4 * g2) / 2) = (uint16_t)nib;
+              *(uint16_t*)(st + (32 * ts + r32) * stage_pitch<16 * H>() + 16 * h + 4 * q + 2 * g2) = (uint16_t)nib;
             }
-            if (g2 == 0) p.hq_scale[(int64_t)fr[tt] * (p.N / 32) + col / 32] = (uint8_t)(k + 127);
+            if (g2 == 0 && fr[tt] < p.R) p.hq_scale[(int64_t)fr[tt] * (p.N / 32) + cw / 32 + h] = (uint8_t)(k + 127);
           }
-        }
+        store_staged_rows<16 * H, NS>(st, lane, fr + tb, p.R, p.hq_codes + cw / 2, p.N / 2);
+      }
     } else if (p.hq_mode == 1) {  // FP8 h: one 128-column block per token, split over the WN waves of a row
       float* am = (float*)lds;     // [WN][kBM rows]
       float bm[G::TT];
@@ -438,7 +478,8 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
         float m = rmax[tt][0];
 #pragma unroll
         for (int h = 1; h < H; ++h) m = fmaxf(m, rmax[tt][h]);
-        if (g2 == 0) am[wn * kBM + (kBM / G::WM) * wm + 32 * tt + r32] = max_pair(m);
+        m = max_pair(m);
+        if (g2 == 0) am[wn * kBM + (kBM / G::WM) * wm + 32 * tt + r32] = m;
       }
       __syncthreads();
 #pragma unroll
@@ -452,35 +493,33 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
       for (int tt = 0; tt < G::TT; ++tt) {
         const int k = dsv4::fp8_block_exp(bm[tt]);
         const float inv = dsv4::pow2f(-k);
-        if (fr[tt] < p.R) {
 #pragma unroll
-          for (int h = 0; h < H; ++h)
+        for (int h = 0; h < H; ++h)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
-              *(uint32_t*)(p.hq_codes + (int64_t)fr[tt] * p.N + cw + 32 * h + 8 * q + 4 * g2) =
-                  pk_fp8x4(bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1), inv);
-            }
-          if (g2 == 0)
-#pragma unroll
-            for (int h = 0; h < H; ++h) p.hq_scale[(int64_t)fr[tt] * (p.N / 32) + cw / 32 + h] = (uint8_t)(k + 127);
-        }
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
+            *(uint32_t*)(st + r32 * stage_pitch<32 * H>() + 32 * h + 8 * q + 4 * g2) =
+                pk_fp8x4(bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1), inv);
+          }
+        store_staged_rows<32 * H, 1>(st, lane, fr + tt, p.R, p.hq_codes + cw, p.N);
+        if (wn == 0 && g2 == 0 && fr[tt] < p.R)  // the block's four scale bytes (N, c0: multiples of 128)
+          *(uint32_t*)(p.hq_scale + (int64_t)fr[tt] * (p.N / 32) + c0 / 32) = (uint32_t)(k + 127) * 0x01010101u;
       }
     }
   } else {
     const int cw = c0 + 32 * G::WT * wn;  // this wave's first output column
 #pragma unroll
-    for (int tt = 0; tt < G::TT; ++tt)
-      if (fr[tt] < p.R)
+    for (int tt = 0; tt < G::TT; ++tt) {
 #pragma unroll
-        for (int wt = 0; wt < G::WT; ++wt)
+      for (int wt = 0; wt < G::WT; ++wt)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-            const int r = 4 * q;
-            *(v2u*)(p.out + (int64_t)fr[tt] * p.N + cw + 32 * wt + 8 * q + 4 * g2) =
-                v2u{pk_bf16(acc[tt][wt][r], acc[tt][wt][r + 1]), pk_bf16(acc[tt][wt][r + 2], acc[tt][wt][r + 3])};
-          }
+        for (int q = 0; q < 4; ++q) {
+          const int r = 4 * q;
+          *(v2u*)(st + r32 * stage_pitch<64 * G::WT>() + 64 * wt + 16 * q + 8 * g2) =
+              v2u{pk_bf16(acc[tt][wt][r], acc[tt][wt][r + 1]), pk_bf16(acc[tt][wt][r + 2], acc[tt][wt][r + 3])};
+        }
+      store_staged_rows<64 * G::WT, 1>(st, lane, fr + tt, p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
+    }
   }
 }
 
@@ -642,7 +681,7 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
   }
   wait_loads_barrier<0>();  // every wave is done with the ring
 
-  big_epilogue<G, GATEUP>(p, acc, lds, c0, wm, wn, r32, g2, fr, wr);
+  big_epilogue<G, GATEUP>(p, acc, lds, c0, wm, wn, lane, fr, wr);
 }
 
 
@@ -665,6 +704,7 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
 //                         pass land on distinct bank groups, two tokens per group).
 struct CfgBf {
   static constexpr int BM = 256, NT = 512, NW = 8, WM = 4, WN = 2, TT = 2, WT = 4;
+  static constexpr int LDS_EPI = 80 * 1024;  // LDS the epilogue may use
 };
 namespace bfk {
 constexpr int ACH = 32;                 // 1-KB token chunks per stage
@@ -676,7 +716,7 @@ constexpr int AS_OFF = NB * STAGE;
 constexpr int LDS = AS_OFF + 2 * SCL;
 constexpr int AV = ACH / CfgBf::NW, BV = BCH / CfgBf::NW, L = AV + BV;  // loads per thread per stage
 constexpr int SV = SCL / (CfgBf::NT * 16);                               // per super-stage
-static_assert(LDS <= 160 * 1024, "ring and scale buffers fit the LDS");
+static_assert(LDS <= 160 * 1024 && LDS >= CfgBf::LDS_EPI, "ring and scale buffers fit the LDS");
 static_assert(AV * CfgBf::NW == ACH && BV * CfgBf::NW == BCH && SV * CfgBf::NT * 16 == SCL, "loads per thread");
 static_assert(L * (NB - 1) + SV < 64, "vmcnt holds 6 bits");
 }  // namespace bfk
@@ -870,7 +910,7 @@ __global__ __launch_bounds__(512, 1) void moe_gemm_big_bf16_kernel(Dsv4GemmArgs 
     }
   }
   wait_loads_barrier<0>();  // every wave is done with the ring
-  big_epilogue<G, GATEUP>(p, acc, lds, c0, wm, wn, r32, g2, fr, wr);
+  big_epilogue<G, GATEUP>(p, acc, lds, c0, wm, wn, lane, fr, wr);
 }
 
 }  // namespace

@@ -10,6 +10,17 @@
 
 namespace dsv4 {
 
+// silu(min(g, L)) * clamp(u, +-L) * w for bf16-rounded g, u (deepseek_v4.py:184-187),
+// the one formula of every gate/up epilogue: a token row gets the same h whichever
+// kernel its expert runs on. limit <= 0: no clamps.
+DSV4_DEV float swiglu(float gt, float up, float w, float limit) {
+  if (limit > 0.0f) {
+    up = fminf(fmaxf(up, -limit), limit);
+    gt = fminf(gt, limit);
+  }
+  return gt / (1.0f + expf(-gt)) * up * w;
+}
+
 // act_quant (npu_ops.py:73-104): per-128 block of one row,
 //   amax = max(max|x|, 1e-4); s = 2^ceil(log2(max(amax * fp32(1/448), 2^-126)))
 //   code = e4m3fn(clamp(x / s, +-448)) (RNE); rt = bf16(e4m3(code) * s)
