@@ -36,6 +36,13 @@
 //             [64+16g, 64+16g+16) in bytes 16-31.
 //   scales  : lane (r, g) supplies the E8M0 of logical block g of its row/col.
 //   C       : lane l holds C[4*(l/16)+i][l%16], i = 0..3.
+// The weights are the MFMA's A operand and the activations its B operand (the layouts of
+// the two are the same; the decode gate/up has them the other way, see moe_gemm_block), so accumulator element i of lane (r, g) is weight column 4g + i
+// of the tile for activation row r: a lane holds runs of 4 columns of one row, and stores
+// 8 bytes of bf16 (4 of E4M3, 2 of E2M1) at a time. With the operands the other way a
+// lane held 4 rows of one column and stored single elements, 16 stores per 16-row
+// subtile of the down GEMM instead of 4, four row-index and routing-weight loads
+// instead of one.
 #include <type_traits>
 
 #include "common.h"
@@ -253,7 +260,7 @@ DSV4_DEV v8i b_operand(const BStageT<B8>& b, int t, int ji) {
   }
 }
 
-template <int AFMT, bool B8 = false>
+template <int AFMT, bool B8, bool WROWS>
 DSV4_DEV void compute(v4f* acc, const AStage<AFMT>& a, const BStageT<B8>& b) {
 #pragma unroll
   for (int ji = 0; ji < 2; ++ji) {
@@ -268,8 +275,12 @@ DSV4_DEV void compute(v4f* acc, const AStage<AFMT>& a, const BStageT<B8>& b) {
     for (int t = 0; t < BStageT<B8>::NTB; ++t) {
       const v8i bv = b_operand<B8>(b, t, ji);
       const int sb = (int)((b.s[t] >> (8 * ji)) & 0xffu);
-      acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[t], AFMT == 0 ? 0 : 4, B8 ? 0 : 4, 0,
-                                                                sa, 0, sb);
+      if constexpr (WROWS)
+        acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[t], B8 ? 0 : 4, AFMT == 0 ? 0 : 4, 0,
+                                                                  sb, 0, sa);
+      else
+        acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[t], AFMT == 0 ? 0 : 4, B8 ? 0 : 4, 0,
+                                                                  sa, 0, sb);
     }
   }
 }
@@ -281,7 +292,7 @@ DSV4_DEV void compute(v4f* acc, const AStage<AFMT>& a, const BStageT<B8>& b) {
 // same 8 k's in the same lane positions, which is all the k pairing of the MFMA needs.
 // (The convert decodes nibble 8 to -0, harmless in a product; a scale byte of 255 gives
 // non-finite weights, as the reference's dequant does.)
-template <bool B8>
+template <bool B8, bool WROWS>
 DSV4_DEV void compute_bf16(v4f* acc, const AStage<kAfmtBf16>& a, const BStageT<B8>& b) {
   static_assert(!B8, "bf16 activations meet E2M1 weights only");
   typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -299,8 +310,9 @@ DSV4_DEV void compute_bf16(v4f* acc, const AStage<kAfmtBf16>& a, const BStageT<B
         const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 2);
         const bf16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 3);
         const bf16x8 bw = bf16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.d[ji][m]), bw, acc[t], 0, 0,
-                                                         0);
+        const bf16x8 aw = __builtin_bit_cast(bf16x8, a.d[ji][m]);
+        if constexpr (WROWS) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw, aw, acc[t], 0, 0, 0);
+        else acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw, bw, acc[t], 0, 0, 0);
       }
     }
 }
@@ -315,70 +327,121 @@ DSV4_DEV int64_t a_row(const Dsv4GemmArgs& p, int f) {
   return f < r0 ? (int64_t)(f / p.a_row_div) : (f < p.R ? (int64_t)(f - r0) : 0);
 }
 
-// Epilogue of one 16-row subtile: lane holds rows row0 + 4*g + i (i = 0..3) of
-// column r16 of each of the 4 tiles. Gate/up: hb receives the bf16 h values the
-// SwiGLU produced (tiles t = 0, 1 are intermediate columns col0 + 16 t + r16) and
-// fr the rows' flat indices; h is written unless the caller fuses its quantisation.
+// two floats -> packed bf16 (RNE, NaN -> 0x7fc0 as f32_to_bf16), low half = a
+DSV4_DEV uint32_t pk_bf16(float a, float b) {
+  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+  const uint32_t w = __builtin_bit_cast(uint32_t, v2bf{(__bf16)a, (__bf16)b});
+  return (a != a ? 0x7fc0u : w & 0xffffu) | (b != b ? 0x7fc00000u : w & 0xffff0000u);
+}
+DSV4_DEV float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
+DSV4_DEV float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+
+// maximum of a value over the four lane groups g (lanes r, r + 16, r + 32, r + 48)
+DSV4_DEV float group_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = fmaxf(__int_as_float(a[0]), __int_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return fmaxf(__int_as_float(b[0]), __int_as_float(b[1]));
+}
+
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+// Epilogue of one 16-row subtile: lane (r16, g) holds columns 16 t + 4 g + i (i = 0..3) of
+// tile t for row row0 + r16. Gate/up: hb[t] receives the bf16 h values the SwiGLU produced
+// for intermediate columns col0 + 16 t + 4 g .. + 3 (t = 0, 1), packed in pairs (zero for a
+// padding row), and fr the row's flat index; h is written unless the caller fuses its
+// quantisation.
 template <bool GATEUP, bool SH = false>
 DSV4_DEV void store_tile(const Dsv4GemmArgs& p, const v4f* acc, int row0, int col0, int g, int r16,
                          uint32_t (*hb)[2] = nullptr, int* fr = nullptr) {
+  const int f = p.sorted_ids[row0 + r16];
+  if (fr) *fr = f;
+  if (GATEUP && hb) hb[0][0] = hb[0][1] = hb[1][0] = hb[1][1] = 0u;
+  if (f >= p.R) return;
+  uint16_t* orow = p.out + (int64_t)f * p.N + col0 + 4 * g;
+  if (GATEUP) {
+    // deepseek_v4.py:177-187: bf16 GEMM outputs -> fp32, clamp, silu(gate) * up * w
+    // (shared-expert rows: w = 1, model_npu.py:478-489 applies no weight)
+    const float w = (!SH || f < p.R - p.shared_a_rows) ? p.topk_w[f] : 1.0f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      uint32_t h2[2];
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        const uint32_t gu0 = pk_bf16(acc[t][i], acc[t + 2][i]), gu1 = pk_bf16(acc[t][i + 1], acc[t + 2][i + 1]);
+        h2[i >> 1] = pk_bf16(dsv4::swiglu(bf16_lo(gu0), bf16_hi(gu0), w, p.swiglu_limit),
+                             dsv4::swiglu(bf16_lo(gu1), bf16_hi(gu1), w, p.swiglu_limit));
+        if (hb) hb[t][i >> 1] = h2[i >> 1];
+      }
+      if (!p.hq_skip_h) *(u32x2_t*)(orow + 16 * t) = u32x2_t{h2[0], h2[1]};
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < kNT; ++t)
+      *(u32x2_t*)(orow + 16 * t) = u32x2_t{pk_bf16(acc[t][0], acc[t][1]), pk_bf16(acc[t][2], acc[t][3])};
+  }
+}
+
+// Gate/up epilogue of one 16-row subtile with the activations as the MFMA's first operand:
+// lane (r16, g) holds rows row0 + 4 g + i (i = 0..3) of column r16 of each tile. Writes h.
+template <bool SH>
+DSV4_DEV void store_tile_columns(const Dsv4GemmArgs& p, const v4f* acc, int row0, int col0, int g, int r16) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int f = p.sorted_ids[row0 + 4 * g + i];
-    if (fr) fr[i] = f;
     if (f >= p.R) continue;
     uint16_t* orow = p.out + (int64_t)f * p.N + col0 + r16;
-    if (GATEUP) {
-      // deepseek_v4.py:177-187: bf16 GEMM outputs -> fp32, clamp, silu(gate) * up * w
-      // (shared-expert rows: w = 1, model_npu.py:478-489 applies no weight)
-      const float w = (!SH || f < p.R - p.shared_a_rows) ? p.topk_w[f] : 1.0f;
+    const float w = (!SH || f < p.R - p.shared_a_rows) ? p.topk_w[f] : 1.0f;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const float gt = dsv4::bf16_to_f32(dsv4::f32_to_bf16(acc[t][i]));
-        const float up = dsv4::bf16_to_f32(dsv4::f32_to_bf16(acc[t + 2][i]));
-        const float h = dsv4::swiglu(gt, up, w, p.swiglu_limit);
-        const uint32_t b = dsv4::f32_to_bf16(h);
-        if (hb) hb[i][t] = b;
-        if (!p.hq_skip_h) orow[16 * t] = (uint16_t)b;
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < kNT; ++t) orow[16 * t] = (uint16_t)dsv4::f32_to_bf16(acc[t][i]);
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t gu = pk_bf16(acc[t][i], acc[t + 2][i]);
+      orow[16 * t] = (uint16_t)dsv4::f32_to_bf16(dsv4::swiglu(bf16_lo(gu), bf16_hi(gu), w, p.swiglu_limit));
     }
   }
 }
 
-// MXFP4 quantisation of the h subtile a gate/up wave holds: its 32 intermediate
-// columns are exactly one 32-element block of each row, spread over the 16
-// lanes of lane group g (2 values each). Same arithmetic as mxfp4_quant_group.
-DSV4_DEV void quantise_h_mxfp4(const Dsv4GemmArgs& p, const uint32_t (*hb)[2], const int* fr, int col0, int g,
-                               int r16) {
-  (void)g;
+// largest magnitude of the 8 values of hb
+DSV4_DEV float h_absmax(const uint32_t (*hb)[2]) {
+  float m = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float v0 = dsv4::bf16_to_f32(hb[i][0]), v1 = dsv4::bf16_to_f32(hb[i][1]);
-    const float amax = dsv4::row16_max(fmaxf(fabsf(v0), fabsf(v1)));
-    const int k = dsv4::mxfp4_block_exp(amax, p.hq_rule);
-    const float inv = dsv4::pow2f(-k);
-    const float y0 = dsv4::mxfp4_clamped(v0, inv, p.hq_rule), y1 = dsv4::mxfp4_clamped(v1, inv, p.hq_rule);
-    const uint32_t own = dsv4::e2m1_pair<0>(0u, y0, y1);  // low nibble: tile 0, high: tile 1
-    const uint32_t nbr = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own, 0xb1, 0xf, 0xf, false);  // lane ^ 1
-    const int f = fr[i];
-    if (f < p.R) {
-      uint8_t* row = p.hq_codes + (int64_t)f * (p.N / 2) + col0 / 2;
-      if ((r16 & 1) == 0) {  // low nibble = even column
-        row[r16 / 2] = (uint8_t)((own & 0xfu) | (nbr << 4));
-        row[8 + r16 / 2] = (uint8_t)((own >> 4) & 0xfu) | (uint8_t)(nbr & 0xf0u);
-      }
-      if (r16 == 0) p.hq_scale[(int64_t)f * (p.N / 32) + col0 / 32] = (uint8_t)(k + 127);
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) m = fmaxf(m, fmaxf(fabsf(bf16_lo(hb[t][j])), fabsf(bf16_hi(hb[t][j]))));
+  return m;
+}
+
+// MXFP4 quantisation of the h subtile a gate/up wave holds: its 32 intermediate
+// columns are exactly one 32-element block of each row, spread over the four lane
+// groups of the row's lane (8 values each). Same arithmetic as mxfp4_quant_loaded.
+DSV4_DEV void quantise_h_mxfp4(const Dsv4GemmArgs& p, const uint32_t (*hb)[2], int f, int col0, int g) {
+  const int k = dsv4::mxfp4_block_exp(group_max(h_absmax(hb)), p.hq_rule);
+  const float inv = dsv4::pow2f(-k);
+  if (f >= p.R) return;
+  uint8_t* row = p.hq_codes + (int64_t)f * (p.N / 2) + col0 / 2 + 2 * g;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    float y[4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      y[2 * j] = dsv4::mxfp4_clamped(bf16_lo(hb[t][j]), inv, p.hq_rule);
+      y[2 * j + 1] = dsv4::mxfp4_clamped(bf16_hi(hb[t][j]), inv, p.hq_rule);
     }
+    *(uint16_t*)(row + 8 * t) = (uint16_t)dsv4::e2m1_pair<1>(dsv4::e2m1_pair<0>(0u, y[0], y[1]), y[2], y[3]);
   }
+  if (g == 0) p.hq_scale[(int64_t)f * (p.N / 32) + col0 / 32] = (uint8_t)(k + 127);
 }
 
 // NTW: the block's routed weights are MFMA-tiled and loaded non-temporally.
 template <int AFMT, bool GATEUP, int NST, bool SH, bool NTW>
 __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& p, const int mb, const int e) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // Which operand the weights are (store_tile / store_tile_columns): with the weights
+  // first a lane holds 4 columns of one row. A decode block holds one or two routed rows
+  // in 16, so for a gate/up that only applies the SwiGLU that form leaves 8 values to each
+  // of the few lanes whose row is real, where the other spreads a row over 16 lanes: 14.0
+  // against 15.2 us at one token, 57.4 in both at 8. The down GEMM (188 -> 187 us at 203
+  // tokens) and the gate/up that quantises whole 32-column blocks of h (332 -> 330) take it.
+  constexpr bool kWRows = !GATEUP || AFMT == 1;
   // the shared expert's blocks carry id shared_expert and read its E4M3 weights
   const bool shared = SH && e == p.shared_expert;
   const Dsv4ExpertPtrs ex = shared ? p.shared : p.experts[e];
@@ -463,10 +526,10 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
 #pragma unroll
       for (int t = 0; t < NTB; ++t) b[j % RING].s[t] = stage_scales<NST>(bs_row[t], j, r16, g);
       if constexpr (AFMT == kAfmtBf16) {
-        compute_bf16<B8>(acc + t0, a[j % RING], b[j % RING]);
+        compute_bf16<B8, kWRows>(acc + t0, a[j % RING], b[j % RING]);
       } else {
         a[j % RING].s = stage_scales<NST>(as_row, j, r16, g);
-        compute<AFMT, B8>(acc + t0, a[j % RING], b[j % RING]);
+        compute<AFMT, B8, kWRows>(acc + t0, a[j % RING], b[j % RING]);
       }
       if constexpr (P > 0) __builtin_amdgcn_sched_barrier(0);
     }
@@ -489,13 +552,15 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
     }
   }
 
-  if (GATEUP && p.hq_mode == 2) {  // MXFP4 h: this wave holds whole 32-column blocks
-    uint32_t hb[4][2];
-    int fr[4];
-    store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, hb, fr);
-    quantise_h_mxfp4(p, hb, fr, col0, g, r16);
-  } else {
+  if (GATEUP && kWRows && p.hq_mode == 2) {  // MXFP4 h: this wave holds whole 32-column blocks
+    uint32_t hb[2][2];
+    int f;
+    store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, hb, &f);
+    quantise_h_mxfp4(p, hb, f, col0, g);
+  } else if constexpr (kWRows) {
     store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16);
+  } else {
+    store_tile_columns<SH>(p, acc, mb * kBM, col0, g, r16);
   }
 }
 
@@ -556,9 +621,8 @@ DSV4_DEV void compute_tiled(v4f (*acc)[kNT], const uint8_t* lds, const uint8_t* 
       for (int t = 0; t < BStageT<B8>::NTB; ++t) {
         const v8i bv = b_operand<B8>(b, t, ji);
         const int sb = (int)((b.s[t] >> (8 * ji)) & 0xffu);
-        acc[mt][t0 + t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[mt][t0 + t],
-                                                                           AFMT == 0 ? 0 : 4, B8 ? 0 : 4, 0, sa, 0,
-                                                                           sb);
+        acc[mt][t0 + t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[mt][t0 + t], B8 ? 0 : 4,
+                                                                           AFMT == 0 ? 0 : 4, 0, sb, 0, sa);
       }
     }
   }
@@ -604,7 +668,7 @@ DSV4_DEV void mfma_half_bf16(v4f (*acc)[kNT], const uint8_t* lds, const bf16x8_t
     for (int t = 0; t < kNT; ++t)
 #pragma unroll
       for (int m = 0; m < 4; ++m)
-        acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[m]), bw[t][m],
+        acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[t][m], __builtin_bit_cast(bf16x8_t, a[m]),
                                                              acc[mt][t], 0, 0, 0);
   }
 }
@@ -878,44 +942,43 @@ __attribute__((always_inline)) DSV4_DEV void tiled_block(const Dsv4GemmArgs& p,
   }
 
   if (GATEUP && p.hq_mode) {
-    uint32_t hb[MT][4][2];
-    int fr[MT][4];
+    uint32_t hb[MT][2][2];
+    int fr[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      store_tile<GATEUP, SH>(p, acc[mt], mb * BM + 16 * mt, col0, g, r16, hb[mt], fr[mt]);
+      store_tile<GATEUP, SH>(p, acc[mt], mb * BM + 16 * mt, col0, g, r16, hb[mt], fr + mt);
     if (p.hq_mode == 2) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) quantise_h_mxfp4(p, hb[mt], fr[mt], col0, g, r16);
+      for (int mt = 0; mt < MT; ++mt) quantise_h_mxfp4(p, hb[mt], fr[mt], col0, g);
     } else {
       // FP8 per 128: waves 4b..4b+3 hold the 128 columns of block b of each row;
       // row maxima meet in LDS (the K loop is done with a_lds)
       float* am = (float*)&a_lds[0][0];  // [NW waves][BM rows]
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float m = dsv4::row16_max(
-              fmaxf(fabsf(dsv4::bf16_to_f32(hb[mt][i][0])), fabsf(dsv4::bf16_to_f32(hb[mt][i][1]))));
-          if (r16 == 0) am[wave * BM + 16 * mt + 4 * g + i] = m;
-        }
+      for (int mt = 0; mt < MT; ++mt) {
+        const float m = group_max(h_absmax(hb[mt]));
+        if (g == 0) am[wave * BM + 16 * mt + r16] = m;
+      }
       __syncthreads();
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int mt = 0; mt < MT; ++mt) {
+        const int row = 16 * mt + r16, f = fr[mt];
+        const float* ab = am + (wave & ~3) * BM + row;
+        const float amax = fmaxf(fmaxf(ab[0], ab[BM]), fmaxf(ab[2 * BM], ab[3 * BM]));
+        const int k = dsv4::fp8_block_exp(amax);
+        const float inv = dsv4::pow2f(-k);
+        if (f < p.R) {
+          uint8_t* crow = p.hq_codes + (int64_t)f * p.N + col0 + 4 * g;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = 16 * mt + 4 * g + i, f = fr[mt][i];
-          const float* ab = am + (wave & ~3) * BM + row;
-          const float amax = fmaxf(fmaxf(ab[0], ab[BM]), fmaxf(ab[2 * BM], ab[3 * BM]));
-          const int k = dsv4::fp8_block_exp(amax);
-          const float inv = dsv4::pow2f(-k);
-          if (f < p.R) {
-            uint8_t* crow = p.hq_codes + (int64_t)f * p.N + col0 + r16;
-            crow[0] = (uint8_t)dsv4::fp8_code(dsv4::bf16_to_f32(hb[mt][i][0]), inv);
-            crow[16] = (uint8_t)dsv4::fp8_code(dsv4::bf16_to_f32(hb[mt][i][1]), inv);
-            if ((wave & 3) == 0 && r16 == 0)
-              *(uint32_t*)(p.hq_scale + (int64_t)f * (p.N / 32) + (col0 & ~127) / 32) = (uint32_t)(k + 127) * 0x01010101u;
+          for (int t = 0; t < 2; ++t) {
+            const float y[4] = {bf16_lo(hb[mt][t][0]), bf16_hi(hb[mt][t][0]), bf16_lo(hb[mt][t][1]),
+                                bf16_hi(hb[mt][t][1])};
+            *(uint32_t*)(crow + 16 * t) = dsv4::fp8_codes4(y, inv);
           }
+          if ((wave & 3) == 0 && g == 0)
+            *(uint32_t*)(p.hq_scale + (int64_t)f * (p.N / 32) + (col0 & ~127) / 32) = (uint32_t)(k + 127) * 0x01010101u;
         }
+      }
     }
   } else {
 #pragma unroll

@@ -51,11 +51,6 @@ DSV4_DEV uint32_t fp8_codes4(const float* f, float inv) {
   const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], lo, true);
 }
-DSV4_DEV uint32_t fp8_code(float f, float inv) {
-  const float y = fminf(fmaxf(f * inv, -448.0f), 448.0f);
-  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y, y, 0, false) & 0xffu;
-}
-
 // 8 bf16 of one 16-byte load as floats; returns their largest magnitude
 DSV4_DEV float unpack8(const uint4 v, float* f) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
