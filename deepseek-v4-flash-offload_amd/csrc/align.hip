@@ -59,7 +59,8 @@ __device__ int block_exclusive_scan(int v, int* lds_waves, int* out_total) {
 // first rather than left as the launch's tail). The routed experts follow;
 // the padding sentinel is R + n_shared.
 // write = false: only off_u/off_p (for workgroups that recompute the layout
-// to scatter their own entries).
+// to scatter their own entries). filled: sorted_ids holds the sentinel already.
+// block_expert is written by the scatter (the entry in a block's first slot).
 // hot (optional, chunked align only): experts with at least hot->hot_min rows get
 // their own layout of kHotBlockM-row blocks (hot->sorted_ids / block_expert /
 // num_post_padded) and no blocks in the main layout; off_p then holds -1 - (their
@@ -67,7 +68,7 @@ __device__ int block_exclusive_scan(int v, int* lds_waves, int* out_total) {
 template <int NT>
 __device__ void align_layout(int c, int bad, int R, int E, int block_m, int max_blocks, int n_shared,
                              const Dsv4AlignOut& o, int* off_u, int* off_p, bool write = true,
-                             const Dsv4AlignHot* hot = nullptr) {
+                             bool filled = false, const Dsv4AlignHot* hot = nullptr) {
   constexpr int kWaves = NT / 64;
   __shared__ int scan_tmp[kWaves];
   __shared__ int totals[4];
@@ -100,16 +101,9 @@ __device__ void align_layout(int c, int bad, int R, int E, int block_m, int max_
   const int cap = max_blocks * block_m;
   if (tid < E) {
     if (o.active && c > 0) o.active[oa] = tid;
-    const int b0 = op / block_m, b1 = min((op + padded) / block_m, max_blocks);
-    for (int b = b0; b < b1; ++b) o.block_expert[b] = tid;
-    const int p1 = min(op + padded, cap);
-    for (int p = op + c; p < p1; ++p) o.sorted_ids[p] = pad_id;
-    if (is_hot) {
-      const int cap_h = hot->max_blocks * kHotBlockM;
-      const int h0 = oph / kHotBlockM, h1 = min((oph + padded_h) / kHotBlockM, hot->max_blocks);
-      for (int b = h0; b < h1; ++b) hot->block_expert[b] = tid;
-      const int q1 = min(oph + padded_h, cap_h);
-      for (int q = oph + c; q < q1; ++q) hot->sorted_ids[q] = pad_id;
+    if (!filled) {
+      const int p1 = min(op + padded, cap);
+      for (int p = op + c; p < p1; ++p) o.sorted_ids[p] = pad_id;
     }
   }
   if (hot && tid == 0) {
@@ -175,11 +169,17 @@ __device__ void align_scatter_range(const IdT* __restrict__ ids, const float* __
       if (o.row) o.row[u] = i / K;
       if (op >= 0) {
         const int p = op + r;
-        if (p < max_blocks * block_m) o.sorted_ids[p] = i;
+        if (p < max_blocks * block_m) {
+          o.sorted_ids[p] = i;
+          if (p % block_m == 0) o.block_expert[p / block_m] = e;  // an expert's rows fill its blocks from the front
+        }
         if (o.padded_pos) o.padded_pos[i] = p;
       } else {  // hot layout (only when hot is given: off_p >= 0 otherwise)
         const int q = -1 - op + r;
-        if (q < hot->max_blocks * kHotBlockM) hot->sorted_ids[q] = i;
+        if (q < hot->max_blocks * kHotBlockM) {
+          hot->sorted_ids[q] = i;
+          if (q % kHotBlockM == 0) hot->block_expert[q / kHotBlockM] = e;
+        }
         if (o.padded_pos) o.padded_pos[i] = -1 - q;
       }
     }
@@ -227,11 +227,17 @@ __device__ void align_body(const IdT* __restrict__ ids, const float* __restrict_
 }
 
 // ---- chunked align for many entries: two launches ------------------------
-// (1) per-chunk counts cc[c][E + 1] (slot E: out-of-range ids), in the same
-//     launch as the quantisation of x; (2) every chunk's workgroup derives the
-//     layout and its own per-expert start from cc and scatters its entries, so
-//     the order is the single-workgroup order (expert ascending, flat index
-//     ascending); workgroup 0 writes the layout outputs.
+// (1) per-chunk counts cc[c][E + 1] (slot E: out-of-range ids) and the padding
+//     sentinel into every slot of the layouts, in the same launch as the
+//     quantisation of x; (2) every chunk's workgroup derives the layout and its
+//     own per-expert start from cc and scatters its entries, so the order is the
+//     single-workgroup order (expert ascending, flat index ascending); workgroup
+//     0 writes the layout outputs.
+// Bound by latency: the counts of all chunks, the scans and the scatter follow each
+// other in one workgroup. 1024 threads take a chunk in one round (256 took four, with
+// three barriers each) and share the chunk counts of an expert four ways, and neither
+// the padding nor the blocks' experts are written in per-expert loops (up to 255 stores
+// by one thread): 39 -> 18 us at 131,072 entries, 33 -> 14 at 16,384, 17.5 -> 8.8 at 4072.
 constexpr int kAlignChunk = 1024;  // entries per chunk
 
 template <typename IdT, int NT>
@@ -251,10 +257,15 @@ __device__ void align_count_chunk(const IdT* __restrict__ ids, int R, int E, int
 
 template <typename IdT, int NT, int QF, int U>
 __global__ __launch_bounds__(NT) void align_count_quant_kernel(const IdT* __restrict__ ids, int R, int E, int C,
-                                                               int* __restrict__ cc, const uint4* __restrict__ x,
+                                                               int* __restrict__ cc, int* __restrict__ slots,
+                                                               int n_slots, int* __restrict__ slots_h, int n_slots_h,
+                                                               int pad_id, const uint4* __restrict__ x,
                                                                int64_t n_groups, int rule, void* q_codes,
                                                                void* q_scale) {
   if ((int)blockIdx.x < C) {
+    const int64_t i0 = (int64_t)blockIdx.x * NT + threadIdx.x, step = (int64_t)C * NT;
+    for (int64_t i = i0; i < n_slots; i += step) slots[i] = pad_id;
+    for (int64_t i = i0; i < n_slots_h; i += step) slots_h[i] = pad_id;
     align_count_chunk<IdT, NT>(ids, R, E, blockIdx.x, cc);
     return;
   }
@@ -281,28 +292,43 @@ __global__ __launch_bounds__(NT) void align_scatter_kernel(const IdT* __restrict
   int* off_p = off_u + E;            // [E]
   int* running = off_p + E;          // [E + 1]
   int* wcount = running + (E + 1);   // [kWaves][E + 1]
-  __shared__ int bad;
   const int c = blockIdx.x, tid = threadIdx.x;
-  int tot = 0;  // count of expert tid
-  for (int e = tid; e <= E; e += NT) {
+  // counts of expert e (slot E: out-of-range ids) in the chunks before c and in all: P
+  // threads per expert, each over every P-th group of 8 chunks (8 loads in flight)
+  const int P = NT / (E + 1) > 4 ? 4 : NT / (E + 1) > 1 ? NT / (E + 1) : 1;
+  int* sum_before = wcount;              // [P][E + 1]
+  int* sum_all = wcount + P * (E + 1);   // [P][E + 1]
+  for (int i = tid; i < P * (E + 1); i += NT) {
+    const int e = i % (E + 1);
     int before = 0, all = 0;
-    for (int c0 = 0; c0 < C; c0 += 16) {  // 16 independent loads in flight
-      int v[16];
+    for (int c0 = 8 * (i / (E + 1)); c0 < C; c0 += 8 * P) {
+      int v[8];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) v[j] = c0 + j < C ? cc[(int64_t)(c0 + j) * (E + 1) + e] : 0;
+      for (int j = 0; j < 8; ++j) v[j] = c0 + j < C ? cc[(int64_t)(c0 + j) * (E + 1) + e] : 0;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
+      for (int j = 0; j < 8; ++j) {
         before += c0 + j < c ? v[j] : 0;
         all += v[j];
       }
     }
+    sum_before[i] = before;
+    sum_all[i] = all;
+  }
+  __syncthreads();
+  int tot = 0, bad = 0;  // count of expert tid; out-of-range ids
+  for (int q = 0; q < P; ++q) bad += sum_all[q * (E + 1) + E];
+  for (int e = tid; e <= E; e += NT) {
+    int before = 0, all = 0;
+    for (int q = 0; q < P; ++q) {
+      before += sum_before[q * (E + 1) + e];
+      all += sum_all[q * (E + 1) + e];
+    }
     running[e] = before;
     if (e == tid) tot = all;
-    if (e == E) bad = all;  // slot E: out-of-range ids
   }
-  for (int i = tid; i < kWaves * (E + 1); i += NT) wcount[i] = 0;
   __syncthreads();
-  align_layout<NT>(tid < E ? tot : 0, bad, R, E, block_m, max_blocks, n_shared, o, off_u, off_p, c == 0, hp);
+  for (int i = tid; i < kWaves * (E + 1); i += NT) wcount[i] = 0;
+  align_layout<NT>(tid < E ? tot : 0, bad, R, E, block_m, max_blocks, n_shared, o, off_u, off_p, c == 0, true, hp);
   align_scatter_range<IdT, NT>(ids, topk_w, c * kAlignChunk, min(R, (c + 1) * kAlignChunk), K, E, block_m,
                                max_blocks, off_u, off_p, running, wcount, o, false, 0, hp);
 }
@@ -364,11 +390,14 @@ __global__ __launch_bounds__(NT) void route_align_quant_kernel(RouteTopkArgs ra,
 
 }  // namespace
 
+// Threads of the one-workgroup align: 256 for small decode batches (fewer waves to
+// synchronise), 1024 above 512 entries (fewer sequential rounds: 10.3 -> 7.4 us at 800
+// entries, 14.8 -> 10.0 at 1624) or 256 experts.
+static bool align_small(int R, int E) { return E <= 256 && R <= 512; }
+
 hipError_t launch_moe_align(const void* topk_ids, int ids_int64, const float* topk_w, int R, int K, int E,
                             int block_m, int max_blocks, const Dsv4AlignOut& o, hipStream_t st) {
-  // small problems (decode) run on 4 waves: fewer waves to synchronise; larger
-  // ones (prefill, or E > 256) on 16 waves: fewer sequential 1024-entry chunks
-  const bool small = E <= 256 && R <= 2048;
+  const bool small = align_small(R, E);
   const int nwaves = small ? 4 : 16;
   const size_t lds = sizeof(int) * (size_t)((E + 1) + E + E + (E + 1) + nwaves * (E + 1));
   if (small) {
@@ -393,7 +422,7 @@ hipError_t launch_moe_align_quant(const void* topk_ids, int ids_int64, const flo
                                   int block_m, int max_blocks, const Dsv4AlignOut& o, const uint16_t* x,
                                   int64_t n_elems, int qfmt, int rule, void* q_codes, void* q_scale,
                                   hipStream_t st, int n_shared) {
-  const bool small = E <= 256 && R <= 2048;
+  const bool small = align_small(R, E);
   const int nt = small ? 256 : 1024;
   const size_t lds = sizeof(int) * (size_t)((E + 1) + E + E + (E + 1) + (nt / 64) * (E + 1));
   const int64_t n_groups = n_elems / 8;
@@ -431,12 +460,14 @@ hipError_t launch_moe_align_chunked(const void* topk_ids, int ids_int64, const f
   constexpr int NT1 = 256;
   const int U = quant_groups_per_thread(n_groups);
   const int64_t qwg = (n_groups + NT1 * U - 1) / (NT1 * U);
-  if (C + qwg > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (C + qwg > 0x7fffffffLL || (int64_t)max_blocks * block_m > 0x7fffffffLL) return hipErrorInvalidValue;
+  const int n_slots = max_blocks * block_m, n_slots_h = hv.hot_min > 0 ? hv.max_blocks * kHotBlockM : 0;
   const dim3 g1((unsigned)(C + qwg));
   const size_t lds1 = sizeof(int) * (size_t)(E + 1);
 #define DSV4_CQU(IDT, QF, U_)                                                                                    \
   hipLaunchKernelGGL((align_count_quant_kernel<IDT, NT1, QF, U_>), g1, dim3(NT1), lds1, st, (const IDT*)topk_ids, \
-                     R, E, C, cc, (const uint4*)x, n_groups, rule, q_codes, q_scale)
+                     R, E, C, cc, o.sorted_ids, n_slots, hv.sorted_ids, n_slots_h, R + n_shared, (const uint4*)x,   \
+                     n_groups, rule, q_codes, q_scale)
 #define DSV4_CQ(IDT, QF) if (U == 2) DSV4_CQU(IDT, QF, 2); else DSV4_CQU(IDT, QF, 1)
   const int qf = x ? qfmt : 2;  // 2: count only
   if (ids_int64) {
@@ -448,16 +479,13 @@ hipError_t launch_moe_align_chunked(const void* topk_ids, int ids_int64, const f
 #undef DSV4_CQU
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // the layout needs one thread per expert: 256 threads up to 256 experts, 1024 above
-#define DSV4_SC(IDT, NT)                                                                                       \
-  hipLaunchKernelGGL((align_scatter_kernel<IDT, NT>), dim3(C), dim3(NT),                                      \
-                     sizeof(int) * (size_t)(E + E + (E + 1) + (NT / 64) * (E + 1)), st, (const IDT*)topk_ids, \
+  // 1024 threads: one per entry of a chunk, and at least one per expert for the layout
+  constexpr int NT2 = 1024;
+#define DSV4_SC(IDT)                                                                                              \
+  hipLaunchKernelGGL((align_scatter_kernel<IDT, NT2>), dim3(C), dim3(NT2),                                        \
+                     sizeof(int) * (size_t)(E + E + (E + 1) + (NT2 / 64) * (E + 1)), st, (const IDT*)topk_ids, \
                      topk_w, R, K, E, C, block_m, max_blocks, n_shared, cc, o, hv)
-  if (E <= 256) {
-    if (ids_int64) DSV4_SC(long long, 256); else DSV4_SC(int32_t, 256);
-  } else {
-    if (ids_int64) DSV4_SC(long long, 1024); else DSV4_SC(int32_t, 1024);
-  }
+  if (ids_int64) DSV4_SC(long long); else DSV4_SC(int32_t);
 #undef DSV4_SC
   return hipGetLastError();
 }

@@ -52,6 +52,18 @@ def test_moe_align_matches_oracle(gpu, T, K, E, bm):
     assert np.array_equal(al["counts"], torch.bincount(flat, minlength=E).numpy())
 
 
+# 512 / 513 entries (256 / 1024 threads), 2048 / 2049 (one workgroup / chunks), a last chunk of one
+# entry, and expert counts that share the chunk sums over 4, 3, 2 and 1 threads
+@pytest.mark.parametrize("T,K,E,bm", [(128, 4, 256, 16), (171, 3, 256, 16), (256, 8, 64, 64), (2049, 1, 16, 64),
+                                      (1025, 9, 255, 64), (1366, 3, 256, 64), (4097, 2, 400, 64), (3073, 1, 511, 16)])
+def test_moe_align_launch_edges(gpu, T, K, E, bm):
+    ids = synth.zipf_topk(T, K, E, synth.rank_permutation(E, 3), np.random.default_rng(T))
+    w = synth.routing_weights(T, K, 5)
+    res = ops.moe_align(torch.from_numpy(ids).to(torch.int32).to(gpu), torch.from_numpy(w).to(gpu), E, bm)
+    torch.cuda.synchronize()
+    _check_align(res, RT.moe_align(ids, w, E, bm), T, K)
+
+
 def test_moe_align_all_to_one_expert_and_out_of_range(gpu):
     ids = np.full((100, 4), 7, dtype=np.int64)
     ids[:, 1] = 3
