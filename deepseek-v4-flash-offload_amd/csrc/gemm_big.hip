@@ -546,6 +546,13 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
   const int wrow_bytes = p.Kdim / 2, srow = p.Kdim / 32;
   const int c0 = nt * (GATEUP ? 128 : 256);  // first intermediate column / output row of W2
   const int slot0 = mb * kHB + (hb % G::WGS) * kBM;
+  // Padding costs nothing where it fills whole workgroups or waves: a half block without a
+  // routed row ends here (half of the hot experts have one), and a wave without one takes
+  // its share of the loads and barriers below but no reads, MFMAs or epilogue.
+  if constexpr (G::WGS == 2) {
+    static_assert(kBM == 128, "two rows per lane");
+    if (__ballot(p.sorted_ids[slot0 + lane] < p.R || p.sorted_ids[slot0 + 64 + lane] < p.R) == 0) return;
+  }
 
   // this lane's A piece per A load (stage 0): chunk wave * AV + v
   const uint8_t* a_src[C::AV];
@@ -605,6 +612,10 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
     fr[tt] = p.sorted_ids[slot0 + (kBM / G::WM) * wm + 32 * tt + r32];
     wr[tt] = GATEUP && fr[tt] < p.R ? p.topk_w[fr[tt]] : 0.0f;
   }
+  bool live_row = false;
+#pragma unroll
+  for (int tt = 0; tt < G::TT; ++tt) live_row |= fr[tt] < p.R;
+  const bool wave_live = __ballot(live_row) != 0;
   // first weight row of this wave's 32-row tile nt in the block
   // gate/up: tiles h < H = gate rows 32 (H wn + h).., tiles H + h = the matching up
   // rows 128 + 32 (H wn + h)..; down: output rows 32 (WT wn + nt)..
@@ -645,6 +656,19 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
 #pragma unroll
     for (int t = 0; t < C::NB; ++t) big_dma_stage<AFMT, HALF>(lds + t * C::STAGE, a_src, b_src, wave, bj, bg, t);
     wait_loads_barrier<C::L * (C::NB - 1)>();
+    if (!wave_live) {  // the loads and barriers of the loop below, one for one
+      int dslot = 0;
+#pragma unroll 1
+      for (int ss = 0; ss < NSS; ++ss) {
+        big_dma_scales<AFMT, HALF>(lds, (ss + 1) & 1, sc_src, wave, min(ss + 1, NSS - 1));
+#pragma unroll 1
+        for (int s = kSS * ss; s < kSS * (ss + 1); ++s) {
+          wait_loads_barrier<C::L * (C::NB - 2)>();
+          big_dma_stage<AFMT, HALF>(lds + dslot * C::STAGE, a_src, b_src, wave, bj, bg, min(s + C::NB, NST - 1));
+          dslot = dslot + 1 == C::NB ? 0 : dslot + 1;
+        }
+      }
+    } else {
     BigFrag<AFMT, HALF> f0, f1;
     BigScl<AFMT, HALF> sr;   // raw scales of the next group of four stages
     BigSclW<AFMT, HALF> sw;  // this lane's scale words of the current group
@@ -681,9 +705,13 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
         step(I3{}, s + 3, f1, f0);
       }
     }
+    }
   }
   wait_loads_barrier<0>();  // every wave is done with the ring
-
+  if (!wave_live) {
+    if (GATEUP && p.hq_mode == 1) __syncthreads();  // the epilogue's one barrier
+    return;
+  }
   big_epilogue<G, GATEUP>(p, acc, lds, c0, wm, wn, lane, fr, wr);
 }
 
@@ -804,6 +832,10 @@ __global__ __launch_bounds__(512, 1) void moe_gemm_big_bf16_kernel(Dsv4GemmArgs 
     fr[tt] = p.sorted_ids[slot0 + (kBM / G::WM) * wm + 32 * tt + r32];
     wr[tt] = GATEUP && fr[tt] < p.R ? p.topk_w[fr[tt]] : 0.0f;
   }
+  bool live_row = false;
+#pragma unroll
+  for (int tt = 0; tt < G::TT; ++tt) live_row |= fr[tt] < p.R;
+  const bool wave_live = __ballot(live_row) != 0;
   constexpr int H = G::WT / 2;
   int brow0[G::WT];
 #pragma unroll
@@ -851,6 +883,10 @@ __global__ __launch_bounds__(512, 1) void moe_gemm_big_bf16_kernel(Dsv4GemmArgs 
       const int boff = (sl >> 2) * bj + (sl & 3) * bg;
 #pragma unroll
       for (int v = 0; v < bfk::BV; ++v) dma16(b_src[v] + boff, fs + (bfk::ACH + wave * bfk::BV + v) * 1024);
+      if (!wave_live) {  // no routed row: loads and barriers only
+        fill = fill + 1 == bfk::NB ? 0 : fill + 1;
+        return;
+      }
       const uint8_t* Ls = lds + slot * bfk::STAGE;
       const uint8_t* S = lds + bfk::AS_OFF + ((s / kSS) & 1) * bfk::SCL;
       if (I == 0) {
@@ -913,6 +949,7 @@ __global__ __launch_bounds__(512, 1) void moe_gemm_big_bf16_kernel(Dsv4GemmArgs 
     }
   }
   wait_loads_barrier<0>();  // every wave is done with the ring
+  if (!wave_live) return;   // (hq_mode is 0: no barrier in the epilogue)
   big_epilogue<G, GATEUP>(p, acc, lds, c0, wm, wn, lane, fr, wr);
 }
 
