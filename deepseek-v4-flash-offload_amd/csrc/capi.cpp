@@ -418,22 +418,22 @@ struct LayerWs {
 // Experts with at least hot_rows_threshold() routed rows run in 256-row blocks on
 // the large-tile kernel in layers of at least hot_layer_rows() routed rows; the rest
 // keep 64-row blocks. Measured with Zipf(1.1) routing over 256 experts (hidden 4096,
-// inter 2048), top-8:
-//   a4w4 (one 8-wave workgroup per hot block): the split lost 5-10 % at 2048 tokens
-//   (the hot experts' blocks too few to fill a launch of their own) and gained 5.5 %
-//   at 4096 tokens with a 256-row threshold (2 % ahead of 128); from 8192 tokens a
-//   128-row threshold was 2-3 % faster than 256.
-//   bf16 (two half-block workgroups per hot block, twice the workgroups per launch):
-//   with a 128-row threshold the split gained 1.5-2 % at 2048 and 4096 tokens, where a
-//   256-row threshold lost 1 % and 0.5-1.5 % against it.
-//   a4w4 below 32,768 rows, where the large-tile launch takes half blocks as well and
-//   runs beside the tiled one: a 128-row threshold gained 3 % at 2048 tokens (1.011-1.018
-//   -> 0.981-0.984 ms), 256 lost 4 %.
-//   pure bf16 (bf16 large-tile kernel, whole blocks, 128-row threshold): layer ms with
-//   / without the split at 2048 tokens 1.682-1.689 / 1.570, 4096 2.588-2.604 / 2.451,
-//   8192 4.087-4.096 / 4.106-4.112, 16384 7.20-7.33 / 7.41; bf16 MFMAs take the same
-//   time on either kernel per useful FLOP until the hot experts fill many whole blocks,
-//   so the pure variant splits from 65,536 routed rows.
+// inter 2048), top-8, layer us with a threshold of 64 / 96 / 128 / 256 rows:
+//   bf16, 2048 tokens 898 / 890 / 870 / -, 4096 1276 / 1265 / 1266 / -, 4500 1360 / 1355 /
+//   1354 / -, 5000 1449 / 1457 / 1468 / -, 6400 1708 / 1740 / 1768 / -, 16384 3590 / 3658 /
+//   3722 / 3792 (192 rows); 48 rows 3606 there.
+//   a4w4, 2048 tokens 847 / 851 / 814 / 839, 4096 1141 / 1125 / 1130 / 1142, 4500 1212 /
+//   1209 / 1197 / -, 5000 1270 / 1285 / 1281 / -, 6007 1421 / 1462 / 1458 / 1472, 16384 3042 /
+//   3109 / 3153 / 3253.
+// So 128 rows, and 64 from 40,000 routed rows, where the smaller experts' workgroups no
+// longer lengthen the launch by a round of their own.
+//   From 16,384 routed rows: splitting at 600, 1024 and 1500 tokens with 128 (64) rows
+//   gave 653 (652), 734 (721), 777 (771) against 663, 717, 791 without (bf16), 645 (634),
+//   710 (693), 743 (730) against 635, 682, 744 (a4w4).
+//   pure bf16 (bf16 large-tile kernel, whole blocks, 128-row threshold): with / without the
+//   split at 2048 tokens 1280 / 1208, 4096 2039 / 1966, 6400 2893 / 2870; 8192 and more gain
+//   (threshold 64 / 96 / 128 / 256 at 16384: 6772 / 6767 / 6677 / 6721), so the pure variant
+//   splits from 65,536 routed rows.
 // DSV4_HOT_LAYER_ROWS and DSV4_HOT_ROWS (0: never) override them, read once.
 static int64_t hot_layer_rows(bool pure) {
   static const int64_t v = [] {
@@ -443,12 +443,12 @@ static int64_t hot_layer_rows(bool pure) {
   return v >= 0 ? v : pure ? 65536 : 16384;
 }
 
-static int hot_rows_threshold(int64_t R, bool fp8) {
+static int hot_rows_threshold(int64_t R, bool pure) {
   static const int v = [] {
     const char* s = getenv("DSV4_HOT_ROWS");
     return s ? atoi(s) : -1;
   }();
-  return v >= 0 ? v : (fp8 || R < 32768 || R >= 65536 ? 128 : 256);
+  return v >= 0 ? v : (!pure && R >= 40000 ? 64 : 128);
 }
 
 // Rows per M block: 16 (decode kernel, ~1-4 rows per active expert) below 2048
@@ -483,7 +483,7 @@ static LayerWs layer_ws(int T, int K, int E, int D, int I, int profile, bool sha
   w.out = take(2 * Rt * D);
   w.align_scratch = R > kAlignSmallRows ? take(align_chunked_scratch_bytes((int)R, E)) : 0;
   w.route_part = routed ? take(dsv4_moe_route_workspace_bytes(T, D, E)) : -1;  // router partial logits
-  const int hot = hot_rows_threshold(R, fp8 || pure);
+  const int hot = hot_rows_threshold(R, pure);
   if (R >= hot_layer_rows(pure) && R > kAlignSmallRows && hot > 0 && moe_gemm_big_supported(D, I, true) &&
       moe_gemm_big_supported(I, D, false)) {
     w.hot_min = hot;

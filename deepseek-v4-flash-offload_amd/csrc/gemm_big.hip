@@ -7,15 +7,9 @@
 // LDS - the A rows gathered through sorted_ids, the weight rows from the
 // expert's slot - so every weight byte a workgroup brings from L2 serves 128 or
 // 256 rows (the 16/64-row kernels re-read an expert's weights once per 16 or 64
-// rows) and every A byte 256 weight rows. Two waves share each SIMD, each with
-// 128 accumulator registers of v_mfma_scale_f32_32x32x64_f8f6f4 tiles, in one of
-// two shapes picked per launch (Cfg):
-//   whole blocks (E2M1 A from 32,768 rows): one workgroup of 8 waves per CU over
-//                    the whole 256-row block; a wave owns 128 rows x 64 weight rows
-//                    (4 x 2 tiles).
-//   half blocks (E4M3 A; E2M1 A below 32,768 rows): two workgroups of 4 waves per
-//                    CU, each over half a block (128 rows); a wave owns 64 rows x
-//                    128 weight rows (2 x 4).
+// rows) and every A byte 256 weight rows. Two workgroups of 4 waves share each CU, each
+// over half a block (128 rows); a wave owns 64 rows x 128 weight rows (2 x 4 tiles of
+// v_mfma_scale_f32_32x32x64_f8f6f4, 128 accumulator registers), two waves per SIMD.
 // A weight fragment read from LDS feeds TT MFMAs and an activation fragment WT.
 // Two waves per SIMD let one wave's MFMAs run while the other waits at a barrier
 // or on its LDS reads (against one 128 x 128 wave per SIMD, 256 accumulators in
@@ -27,7 +21,7 @@
 // Operands move global -> LDS with global_load_lds_dwordx4 (lane i of one
 // instruction writes its 16 bytes at the instruction's LDS base + 16 i): no
 // staging registers, so a ring of NB stage slots keeps NB - 1 stages of loads
-// in flight (96 KB per CU with E2M1 A on whole blocks, 2 x 32-36 KB on half blocks);
+// in flight (2 x 32-36 KB per CU);
 // the depth of the ring, and the second workgroup, hide the load latency.
 // Each 1-KB chunk is laid out in the order the MFMA lanes read it, with an XOR
 // swizzle that puts the 16 lanes of each ds_read_b128 pass on distinct banks.
@@ -65,38 +59,35 @@ constexpr int kBN = 256;     // weight rows per block
 constexpr int kKS = 64;      // k per stage
 constexpr int kSS = 16;      // stages per scale super-stage (1024 k)
 
-// Workgroup shapes. HALF: two workgroups per CU, each half a 256-row block, 4 waves of
-// 64 rows x 128 weight rows; otherwise one workgroup per CU over the whole block, 8
-// waves of 128 x 64. Either way two waves share a SIMD; two independent workgroups let
-// one's MFMAs run while the other waits at its stage barrier. Measured (layer time, same
-// runs): E4M3 at 16384 tokens 4.49-4.60 ms with the 8-wave shape against 4.27-4.29 with
-// the half-block one; E2M1 at 16384 tokens 3.54-3.68 against 3.68-3.76, at 2048 tokens
-// (16,384 routed rows, the hot experts' blocks too few to fill the CUs) 1.012-1.022
-// against 0.981-0.984. launch_moe_gemm_big picks HALF for E4M3, and for E2M1 below
-// 32,768 rows.
-template <int AFMT, bool HALF>
+// Workgroup shape: two workgroups per CU, each half a 256-row block, 4 waves of 64 rows x
+// 128 weight rows; two waves share a SIMD, and two independent workgroups let one's MFMAs
+// run while the other waits at its stage barrier or runs its epilogue, and a half block
+// that holds only padding costs nothing. One workgroup of 8 waves (128 x 64 each) over the
+// whole block measured, layer time in the same runs: E4M3 at 16384 tokens 4.49-4.60 ms
+// against 4.27-4.29 (before padding was skipped); E2M1 with the best threshold of each,
+// 16384 tokens 3.18 ms against 3.04, 6007 tokens 1.486 against 1.421.
 struct Cfg {
-  static constexpr int BM = HALF ? 128 : 256;  // rows per workgroup
-  static constexpr int NT = HALF ? 256 : 512;  // threads
+  static constexpr int BM = 128;               // rows per workgroup
+  static constexpr int NT = 256;               // threads
   static constexpr int NW = NT / 64;           // waves
   static constexpr int WM = 2, WN = NW / WM;   // wave grid over rows x weight rows
   static constexpr int TT = BM / WM / 32;      // 32-row token tiles per wave
   static constexpr int WT = kBN / WN / 32;     // 32-row weight tiles per wave
-  static constexpr int WGS = HALF ? 2 : 1;     // workgroups per CU
+  static constexpr int WGS = 2;                // workgroups per CU, and per block
   static constexpr int LDS_EPI = 72 * 1024;    // LDS the epilogue may use (the ring's, checked below)
 };
 
-template <int AFMT, bool HALF>
+template <int AFMT>
 struct Big {
-  using G = Cfg<AFMT, HALF>;
+  using G = Cfg;
   static constexpr int kBM = G::BM;
   static constexpr int kNT = G::NT;
   static constexpr int ACH = kBM * (AFMT == 0 ? kKS : kKS / 2) / 1024;  // 1-KB A chunks per stage
   static constexpr int BCH = kBN * (kKS / 2) / 1024;  // 1-KB weight chunks per stage
   static constexpr int STAGE = (ACH + BCH) * 1024;
-  static constexpr int NB = HALF ? (AFMT == 0 ? 3 : 4) : (AFMT == 0 ? 5 : 7);  // stage slots of the ring
-  static constexpr int AV = ACH / Cfg<AFMT, HALF>::NW;      // A loads per thread per stage
-  static constexpr int BV = BCH / Cfg<AFMT, HALF>::NW;      // weight loads per thread per stage
+  static constexpr int NB = AFMT == 0 ? 3 : 4;  // stage slots of the ring
+  static constexpr int AV = ACH / Cfg::NW;      // A loads per thread per stage
+  static constexpr int BV = BCH / Cfg::NW;      // weight loads per thread per stage
   static constexpr int L = AV + BV;
   typedef v16f Acc[G::TT][G::WT];  // a wave's accumulators
   // scales: one super-stage = 32 bytes per A row and per weight row (two 16-byte
@@ -108,8 +99,8 @@ struct Big {
   static constexpr int BS_OFF = kBM * 32;            // weight rows within a buffer
   static constexpr int SV = SCL / (kNT * 16);         // scale loads per thread per super-stage
   static constexpr int LDS = NB * STAGE + 2 * SCL;
-  static_assert(LDS * Cfg<AFMT, HALF>::WGS <= 160 * 1024, "the stage ring and two scale super-stages must fit the LDS");
-  static_assert(LDS >= Cfg<AFMT, HALF>::LDS_EPI, "the epilogue's share");
+  static_assert(LDS * Cfg::WGS <= 160 * 1024, "the stage ring and two scale super-stages must fit the LDS");
+  static_assert(LDS >= Cfg::LDS_EPI, "the epilogue's share");
   static_assert(BCH == 8 && (ACH * 1024) == kBM * (AFMT == 0 ? kKS : kKS / 2), "chunking");
   static_assert(AV * G::NW == ACH && BV * G::NW == BCH && SV * kNT * 16 == SCL, "loads per thread");
   static_assert(L * NB + SV < 64, "vmcnt holds 6 bits");
@@ -146,9 +137,9 @@ DSV4_DEV void wait_loads_barrier() {
 
 // Issues the scale loads of super-stage ss into buffer `buf` (sc_src: this lane's
 // pieces at super-stage 0, in load order (wave * SV + v) * 64 + lane).
-template <int AFMT, bool HALF>
+template <int AFMT>
 DSV4_DEV void big_dma_scales(uint8_t* lds, int buf, const uint8_t* const* sc_src, int wave, int ss) {
-  using C = Big<AFMT, HALF>;
+  using C = Big<AFMT>;
 #pragma unroll
   for (int v = 0; v < C::SV; ++v) dma16(sc_src[v] + ss * 32, lds + C::AS_OFF + buf * C::SCL + (wave * C::SV + v) * 1024);
 }
@@ -156,10 +147,10 @@ DSV4_DEV void big_dma_scales(uint8_t* lds, int buf, const uint8_t* const* sc_src
 // Issues stage s's loads into ring slot `slot`: this wave's A chunks wave * AV + v and
 // weight chunks wave * BV + v (a_src / b_src: this lane's piece at stage 0; bj / bg:
 // the weight offset per 4 stages / per stage within them, no branch in the loop).
-template <int AFMT, bool HALF>
+template <int AFMT>
 DSV4_DEV void big_dma_stage(uint8_t* slot, const uint8_t* const* a_src, const uint8_t* const* b_src, int wave,
                             int bj, int bg, int s) {
-  using C = Big<AFMT, HALF>;
+  using C = Big<AFMT>;
   const int aoff = s * (AFMT == 0 ? kKS : kKS / 2);
 #pragma unroll
   for (int v = 0; v < C::AV; ++v) dma16(a_src[v] + aoff, slot + (wave * C::AV + v) * 1024);
@@ -171,24 +162,24 @@ DSV4_DEV void big_dma_stage(uint8_t* slot, const uint8_t* const* a_src, const ui
 
 // The fragments of one stage for this wave: weight tiles nt (16 bytes each), A tiles
 // mt (E4M3: 2 x 16 bytes, E2M1: 16 bytes).
-template <int AFMT, bool HALF>
+template <int AFMT>
 struct BigFrag {
-  v4i b[Cfg<AFMT, HALF>::WT];
-  v4i lo[Cfg<AFMT, HALF>::TT];
-  v4i hi[AFMT == 0 ? Cfg<AFMT, HALF>::TT : 1];
+  v4i b[Cfg::WT];
+  v4i lo[Cfg::TT];
+  v4i hi[AFMT == 0 ? Cfg::TT : 1];
 };
 
 // Reads one stage's fragments from ring slot L. a_lo / a_hi: this lane's byte offsets
 // inside an A chunk, b_lane inside a weight chunk.
-template <int AFMT, bool HALF>
-DSV4_DEV void big_read(BigFrag<AFMT, HALF>& F, const uint8_t* L, int wm, const int* brow0, int r32, int a_lo,
+template <int AFMT>
+DSV4_DEV void big_read(BigFrag<AFMT>& F, const uint8_t* L, int wm, const int* brow0, int r32, int a_lo,
                        int a_hi, int b_lane) {
-  using C = Big<AFMT, HALF>;
+  using C = Big<AFMT>;
 #pragma unroll
-  for (int nt = 0; nt < Cfg<AFMT, HALF>::WT; ++nt) F.b[nt] = *(const v4i*)(L + (C::ACH + brow0[nt] / 32) * 1024 + b_lane);
+  for (int nt = 0; nt < Cfg::WT; ++nt) F.b[nt] = *(const v4i*)(L + (C::ACH + brow0[nt] / 32) * 1024 + b_lane);
 #pragma unroll
-  for (int mt = 0; mt < Cfg<AFMT, HALF>::TT; ++mt) {
-    const int row0 = (Cfg<AFMT, HALF>::BM / Cfg<AFMT, HALF>::WM) * wm + 32 * mt;
+  for (int mt = 0; mt < Cfg::TT; ++mt) {
+    const int row0 = (Cfg::BM / Cfg::WM) * wm + 32 * mt;
     if (AFMT == 0) {
       const uint8_t* ch = L + (row0 / 16 + (r32 >> 4)) * 1024;
       F.lo[mt] = *(const v4i*)(ch + a_lo);
@@ -208,43 +199,43 @@ DSV4_DEV void big_read(BigFrag<AFMT, HALF>& F, const uint8_t* L, int wm, const i
 // per four stages instead of one byte read per tile per stage. Shifted right by 8 g2,
 // stage 4j + i's byte sits at bit 16 (i % 2) of word i / 2, which the MFMA picks with
 // its scale byte select (op_sel = 2 (i % 2)).
-template <int AFMT, bool HALF>
+template <int AFMT>
 struct BigScl {
-  uint64_t b[Cfg<AFMT, HALF>::WT], a[Cfg<AFMT, HALF>::TT];
+  uint64_t b[Cfg::WT], a[Cfg::TT];
 };
-template <int AFMT, bool HALF>
+template <int AFMT>
 struct BigSclW {
-  uint32_t b[Cfg<AFMT, HALF>::WT][2], a[Cfg<AFMT, HALF>::TT][2];
+  uint32_t b[Cfg::WT][2], a[Cfg::TT][2];
 };
 
 // Reads the raw scale groups of stages s0 .. s0 + 3 (s0 % 4 == 0, the stage within its
 // super-stage) from super-stage buffer S.
-template <int AFMT, bool HALF>
-DSV4_DEV void big_read_scales(BigScl<AFMT, HALF>& R, const uint8_t* S, int s0, int wm, const int* brow0, int r32) {
-  constexpr int kBM = Cfg<AFMT, HALF>::BM;
+template <int AFMT>
+DSV4_DEV void big_read_scales(BigScl<AFMT>& R, const uint8_t* S, int s0, int wm, const int* brow0, int r32) {
+  constexpr int kBM = Cfg::BM;
   const int off = 2 * (s0 & 7), half = s0 >> 3;  // byte within the row's 16-byte piece `half`
 #pragma unroll
-  for (int nt = 0; nt < Cfg<AFMT, HALF>::WT; ++nt)
+  for (int nt = 0; nt < Cfg::WT; ++nt)
     R.b[nt] = *(const uint64_t*)(S + kBM * 32 + (half * kBN + brow0[nt] + r32) * 16 + off);
 #pragma unroll
-  for (int mt = 0; mt < Cfg<AFMT, HALF>::TT; ++mt) {
-    const int row0 = (kBM / Cfg<AFMT, HALF>::WM) * wm + 32 * mt;
+  for (int mt = 0; mt < Cfg::TT; ++mt) {
+    const int row0 = (kBM / Cfg::WM) * wm + 32 * mt;
     R.a[mt] = *(const uint64_t*)(S + (half * kBM + row0 + r32) * 16 + off);
   }
 }
 
 // This lane's scale words of a group: its bytes (g2) moved to bits 0, 16 of two words.
-template <int AFMT, bool HALF>
-DSV4_DEV void big_scale_words(BigSclW<AFMT, HALF>& W, const BigScl<AFMT, HALF>& R, int g2) {
+template <int AFMT>
+DSV4_DEV void big_scale_words(BigSclW<AFMT>& W, const BigScl<AFMT>& R, int g2) {
   const int sh = 8 * g2;
 #pragma unroll
-  for (int nt = 0; nt < Cfg<AFMT, HALF>::WT; ++nt) {
+  for (int nt = 0; nt < Cfg::WT; ++nt) {
     const uint64_t v = R.b[nt] >> sh;
     W.b[nt][0] = (uint32_t)v;
     W.b[nt][1] = (uint32_t)(v >> 32);
   }
 #pragma unroll
-  for (int mt = 0; mt < Cfg<AFMT, HALF>::TT; ++mt) {
+  for (int mt = 0; mt < Cfg::TT; ++mt) {
     const uint64_t v = R.a[mt] >> sh;
     W.a[mt][0] = (uint32_t)v;
     W.a[mt][1] = (uint32_t)(v >> 32);
@@ -255,15 +246,15 @@ DSV4_DEV void big_scale_words(BigSclW<AFMT, HALF>& W, const BigScl<AFMT, HALF>& 
 // matrix pipe with FP8 A) followed by one of the stage's loads and two of the next
 // stage's fragment reads, so the LDS and the memory pipe work under the MFMAs and
 // the reads are done long before the next barrier waits for them.
-template <int AFMT, bool HALF, int I>
+template <int AFMT, int I>
 DSV4_DEV void big_sched() {
-  using G = Cfg<AFMT, HALF>;
+  using G = Cfg;
   // ds_reads of big_read (+ big_read_scales in the last stage of a group)
   constexpr int kReads = G::WT + (AFMT == 0 ? 2 : 1) * G::TT + (I == 3 ? G::WT + G::TT : 0);
 #pragma unroll
   for (int i = 0; i < G::TT * G::WT; ++i) {
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                      // MFMA
-    if (i < Big<AFMT, HALF>::L) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
+    if (i < Big<AFMT>::L) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
     if (2 * i < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);    // DS read
   }
 }
@@ -272,15 +263,15 @@ DSV4_DEV void big_sched() {
 // operand and the activations its B operand, so accumulator (tt, wt) holds weight
 // columns x tokens: register r of lane l = weight column 8(r/4) + 4(l/32) + r%4 of
 // weight tile wt, token l%32 of token tile tt (the E4M3 B layout is the A layout).
-template <int AFMT, bool HALF, int I>
-DSV4_DEV void big_mfma(typename Big<AFMT, HALF>::Acc& acc, const BigFrag<AFMT, HALF>& F, const BigSclW<AFMT, HALF>& W) {
+template <int AFMT, int I>
+DSV4_DEV void big_mfma(typename Big<AFMT>::Acc& acc, const BigFrag<AFMT>& F, const BigSclW<AFMT>& W) {
 #pragma unroll
-  for (int tt = 0; tt < Cfg<AFMT, HALF>::TT; ++tt) {
+  for (int tt = 0; tt < Cfg::TT; ++tt) {
     const v4i lo = F.lo[tt];
     const v4i hi = AFMT == 0 ? F.hi[tt] : v4i{0, 0, 0, 0};
     const v8i xf = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
-    for (int wt = 0; wt < Cfg<AFMT, HALF>::WT; ++wt) {
+    for (int wt = 0; wt < Cfg::WT; ++wt) {
       const v8i wf = v8i{F.b[wt].x, F.b[wt].y, F.b[wt].z, F.b[wt].w, 0, 0, 0, 0};
       // stage I of the scale group: word I / 2, byte 2 (I % 2)
       acc[tt][wt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf, xf, acc[tt][wt], 4, AFMT == 0 ? 0 : 4,
@@ -372,25 +363,22 @@ DSV4_DEV void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Stores 32 * NTT staged rows of ROWB bytes (NTT token tiles whose lane r32 holds flat
-// index fr[tile]) to base + f * row_stride; rows with f >= R (padding) are left out.
+// Stores a token tile's 32 staged rows of ROWB bytes (lane r32 holds row r32's flat index
+// f) to base + f * row_stride; rows with f >= R (padding) are left out.
 // Non-temporal: the outputs of the sizes this kernel serves do not stay in the L2 until
 // their reader runs, and leave it to the operands (layer at 16384 tokens 3278 -> 3252 us
 // a4w4, 3812 -> 3800 us bf16; 2048 tokens unchanged).
-template <int ROWB, int NTT>
-DSV4_DEV void store_staged_rows(const uint8_t* st, int lane, const int* fr, int R, uint8_t* base, int64_t row_stride) {
+template <int ROWB>
+DSV4_DEV void store_staged_rows(const uint8_t* st, int lane, int fr, int R, uint8_t* base, int64_t row_stride) {
   constexpr int CPR = ROWB / 16;        // 16-byte pieces per row
   constexpr int RPI = 64 / CPR;         // rows per store instruction
-  constexpr int IT = 32 * NTT / RPI;
-  static_assert(CPR * RPI == 64 && IT * RPI == 32 * NTT, "whole store instructions");
+  constexpr int IT = 32 / RPI;
+  static_assert(CPR * RPI == 64 && IT * RPI == 32, "whole store instructions");
   wave_lds_fence();
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
     const int row = it * RPI + lane / CPR, ch = lane % CPR;
-    const int t0 = it * RPI / 32;
-    int f;
-    if constexpr (RPI == 64) f = lane < 32 ? fr[t0] : fr[t0 + 1];
-    else f = __shfl(fr[t0], row & 31, 64);
+    const int f = __shfl(fr, row, 64);
     const v4i v = *(const v4i*)(st + row * stage_pitch<ROWB>() + 16 * ch);
     if (f < R) __builtin_nontemporal_store(v, (v4i*)(base + (int64_t)f * row_stride + 16 * ch));
   }
@@ -447,31 +435,26 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
           for (int q = 0; q < 4; ++q)
             *(v2u*)(st + r32 * stage_pitch<64 * H>() + 64 * h + 16 * q + 8 * g2) =
                 v2u{hp[tt][h][q][0], hp[tt][h][q][1]};
-        store_staged_rows<64 * H, 1>(st, lane, fr + tt, p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
+        store_staged_rows<64 * H>(st, lane, fr[tt], p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
       }
     }
     if (p.hq_mode == 2) {  // MXFP4 h: one 32-column block per (tt, h), half of it in each lane of a pair
-      constexpr int NS = H == 1 ? 2 : 1;  // token tiles per staged batch (16 H bytes per row)
-      static_assert(G::TT % NS == 0, "whole batches");
 #pragma unroll
-      for (int tb = 0; tb < G::TT; tb += NS) {
+      for (int tt = 0; tt < G::TT; ++tt) {
 #pragma unroll
-        for (int ts = 0; ts < NS; ++ts)
+        for (int h = 0; h < H; ++h) {
+          const int k = dsv4::mxfp4_block_exp(max_pair(rmax[tt][h]), p.hq_rule);
+          const float inv = dsv4::pow2f(-k);
 #pragma unroll
-          for (int h = 0; h < H; ++h) {
-            const int tt = tb + ts;
-            const int k = dsv4::mxfp4_block_exp(max_pair(rmax[tt][h]), p.hq_rule);
-            const float inv = dsv4::pow2f(-k);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
-              const uint32_t nib = pk_fp4x2(bf16_lo(w0), bf16_hi(w0), inv, p.hq_rule) |
-                                   pk_fp4x2(bf16_lo(w1), bf16_hi(w1), inv, p.hq_rule) << 8;
-              *(uint16_t*)(st + (32 * ts + r32) * stage_pitch<16 * H>() + 16 * h + 4 * q + 2 * g2) = (uint16_t)nib;
-            }
-            if (g2 == 0 && fr[tt] < p.R) p.hq_scale[(int64_t)fr[tt] * (p.N / 32) + cw / 32 + h] = (uint8_t)(k + 127);
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
+            const uint32_t nib = pk_fp4x2(bf16_lo(w0), bf16_hi(w0), inv, p.hq_rule) |
+                                 pk_fp4x2(bf16_lo(w1), bf16_hi(w1), inv, p.hq_rule) << 8;
+            *(uint16_t*)(st + r32 * stage_pitch<16 * H>() + 16 * h + 4 * q + 2 * g2) = (uint16_t)nib;
           }
-        store_staged_rows<16 * H, NS>(st, lane, fr + tb, p.R, p.hq_codes + cw / 2, p.N / 2);
+          if (g2 == 0 && fr[tt] < p.R) p.hq_scale[(int64_t)fr[tt] * (p.N / 32) + cw / 32 + h] = (uint8_t)(k + 127);
+        }
+        store_staged_rows<16 * H>(st, lane, fr[tt], p.R, p.hq_codes + cw / 2, p.N / 2);
       }
     } else if (p.hq_mode == 1) {  // FP8 h: one 128-column block per token, split over the WN waves of a row
       float* am = (float*)lds;     // [WN][kBM rows]
@@ -504,7 +487,7 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
             *(uint32_t*)(st + r32 * stage_pitch<32 * H>() + 32 * h + 8 * q + 4 * g2) =
                 pk_fp8x4(bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1), inv);
           }
-        store_staged_rows<32 * H, 1>(st, lane, fr + tt, p.R, p.hq_codes + cw, p.N);
+        store_staged_rows<32 * H>(st, lane, fr[tt], p.R, p.hq_codes + cw, p.N);
         if (wn == 0 && g2 == 0 && fr[tt] < p.R)  // the block's four scale bytes (N, c0: multiples of 128)
           *(uint32_t*)(p.hq_scale + (int64_t)fr[tt] * (p.N / 32) + c0 / 32) = (uint32_t)(k + 127) * 0x01010101u;
       }
@@ -521,15 +504,15 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
           *(v2u*)(st + r32 * stage_pitch<64 * G::WT>() + 64 * wt + 16 * q + 8 * g2) =
               v2u{pk_bf16(acc[tt][wt][r], acc[tt][wt][r + 1]), pk_bf16(acc[tt][wt][r + 2], acc[tt][wt][r + 3])};
         }
-      store_staged_rows<64 * G::WT, 1>(st, lane, fr + tt, p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
+      store_staged_rows<64 * G::WT>(st, lane, fr[tt], p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
     }
   }
 }
 
-template <int AFMT, bool HALF, bool GATEUP>
-__global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void moe_gemm_big_kernel(Dsv4GemmArgs p) {
-  using C = Big<AFMT, HALF>;
-  using G = Cfg<AFMT, HALF>;
+template <int AFMT, bool GATEUP>
+__global__ __launch_bounds__((Cfg::NT), (Cfg::WGS)) void moe_gemm_big_kernel(Dsv4GemmArgs p) {
+  using C = Big<AFMT>;
+  using G = Cfg;
   constexpr int kBM = G::BM, H = G::WT / 2;  // H: gate (and up) tiles per wave of gate/up
   __shared__ __attribute__((aligned(16))) uint8_t lds[C::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -549,10 +532,8 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
   // Padding costs nothing where it fills whole workgroups or waves: a half block without a
   // routed row ends here (half of the hot experts have one), and a wave without one takes
   // its share of the loads and barriers below but no reads, MFMAs or epilogue.
-  if constexpr (G::WGS == 2) {
-    static_assert(kBM == 128, "two rows per lane");
-    if (__ballot(p.sorted_ids[slot0 + lane] < p.R || p.sorted_ids[slot0 + 64 + lane] < p.R) == 0) return;
-  }
+  static_assert(kBM == 128, "two rows per lane");
+  if (__ballot(p.sorted_ids[slot0 + lane] < p.R || p.sorted_ids[slot0 + 64 + lane] < p.R) == 0) return;
 
   // this lane's A piece per A load (stage 0): chunk wave * AV + v
   const uint8_t* a_src[C::AV];
@@ -652,42 +633,42 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
     // flight before storing them (it cannot see that 16 stages have passed). NST =
     // K / 64 is a multiple of 16.
     const int NSS = NST / kSS;
-    big_dma_scales<AFMT, HALF>(lds, 0, sc_src, wave, 0);
+    big_dma_scales<AFMT>(lds, 0, sc_src, wave, 0);
 #pragma unroll
-    for (int t = 0; t < C::NB; ++t) big_dma_stage<AFMT, HALF>(lds + t * C::STAGE, a_src, b_src, wave, bj, bg, t);
+    for (int t = 0; t < C::NB; ++t) big_dma_stage<AFMT>(lds + t * C::STAGE, a_src, b_src, wave, bj, bg, t);
     wait_loads_barrier<C::L * (C::NB - 1)>();
     if (!wave_live) {  // the loads and barriers of the loop below, one for one
       int dslot = 0;
 #pragma unroll 1
       for (int ss = 0; ss < NSS; ++ss) {
-        big_dma_scales<AFMT, HALF>(lds, (ss + 1) & 1, sc_src, wave, min(ss + 1, NSS - 1));
+        big_dma_scales<AFMT>(lds, (ss + 1) & 1, sc_src, wave, min(ss + 1, NSS - 1));
 #pragma unroll 1
         for (int s = kSS * ss; s < kSS * (ss + 1); ++s) {
           wait_loads_barrier<C::L * (C::NB - 2)>();
-          big_dma_stage<AFMT, HALF>(lds + dslot * C::STAGE, a_src, b_src, wave, bj, bg, min(s + C::NB, NST - 1));
+          big_dma_stage<AFMT>(lds + dslot * C::STAGE, a_src, b_src, wave, bj, bg, min(s + C::NB, NST - 1));
           dslot = dslot + 1 == C::NB ? 0 : dslot + 1;
         }
       }
     } else {
-    BigFrag<AFMT, HALF> f0, f1;
-    BigScl<AFMT, HALF> sr;   // raw scales of the next group of four stages
-    BigSclW<AFMT, HALF> sw;  // this lane's scale words of the current group
-    big_read<AFMT, HALF>(f0, lds, wm, brow0, r32, a_lo, a_hi, b_lane);
-    big_read_scales<AFMT, HALF>(sr, lds + C::AS_OFF, 0, wm, brow0, r32);
+    BigFrag<AFMT> f0, f1;
+    BigScl<AFMT> sr;   // raw scales of the next group of four stages
+    BigSclW<AFMT> sw;  // this lane's scale words of the current group
+    big_read<AFMT>(f0, lds, wm, brow0, r32, a_lo, a_hi, b_lane);
+    big_read_scales<AFMT>(sr, lds + C::AS_OFF, 0, wm, brow0, r32);
     int slot = 0;  // ring slot of stage s
     // stage s (I = s % 4 of its scale group): multiply Fc (stage s), read stage s + 1
     // into Fn and, in the group's last stage, the next group's scales
-    auto step = [&](auto I_, int s, BigFrag<AFMT, HALF>& Fc, BigFrag<AFMT, HALF>& Fn) __attribute__((always_inline)) {
+    auto step = [&](auto I_, int s, BigFrag<AFMT>& Fc, BigFrag<AFMT>& Fn) __attribute__((always_inline)) {
       constexpr int I = decltype(I_)::value;
       const int nslot = slot + 1 == C::NB ? 0 : slot + 1;
       wait_loads_barrier<C::L * (C::NB - 2)>();
-      if (I == 0) big_scale_words<AFMT, HALF>(sw, sr, g2);
-      big_dma_stage<AFMT, HALF>(lds + slot * C::STAGE, a_src, b_src, wave, bj, bg, min(s + C::NB, NST - 1));
+      if (I == 0) big_scale_words<AFMT>(sw, sr, g2);
+      big_dma_stage<AFMT>(lds + slot * C::STAGE, a_src, b_src, wave, bj, bg, min(s + C::NB, NST - 1));
       const int s1 = s + 1;
-      big_read<AFMT, HALF>(Fn, lds + nslot * C::STAGE, wm, brow0, r32, a_lo, a_hi, b_lane);
-      if (I == 3) big_read_scales<AFMT, HALF>(sr, lds + C::AS_OFF + ((s1 / kSS) & 1) * C::SCL, s1 % kSS, wm, brow0, r32);
-      big_mfma<AFMT, HALF, I>(acc, Fc, sw);
-      big_sched<AFMT, HALF, I>();
+      big_read<AFMT>(Fn, lds + nslot * C::STAGE, wm, brow0, r32, a_lo, a_hi, b_lane);
+      if (I == 3) big_read_scales<AFMT>(sr, lds + C::AS_OFF + ((s1 / kSS) & 1) * C::SCL, s1 % kSS, wm, brow0, r32);
+      big_mfma<AFMT, I>(acc, Fc, sw);
+      big_sched<AFMT, I>();
       slot = nslot;
     };
     using I0 = std::integral_constant<int, 0>;
@@ -696,7 +677,7 @@ __global__ __launch_bounds__((Cfg<AFMT, HALF>::NT), (Cfg<AFMT, HALF>::WGS)) void
     using I3 = std::integral_constant<int, 3>;
 #pragma unroll 1
     for (int ss = 0; ss < NSS; ++ss) {
-      big_dma_scales<AFMT, HALF>(lds, (ss + 1) & 1, sc_src, wave, min(ss + 1, NSS - 1));
+      big_dma_scales<AFMT>(lds, (ss + 1) & 1, sc_src, wave, min(ss + 1, NSS - 1));
 #pragma unroll 1
       for (int s = kSS * ss; s < kSS * (ss + 1); s += 4) {
         step(I0{}, s, f0, f1);
@@ -960,15 +941,15 @@ bool moe_gemm_big_supported(int kdim, int n, bool gateup) {
   return kdim >= 1024 && kdim % 1024 == 0 && n % (gateup ? 128 : 256) == 0;
 }
 
-template <int AFMT, bool HALF>
+template <int AFMT>
 static void launch_big(const Dsv4GemmArgs& a, bool gateup, int ntiles, hipStream_t st) {
-  using G = Cfg<AFMT, HALF>;
+  using G = Cfg;
   // workgroups' M extent: WGS per hot-layout block, in whole groups of 32 for the XCD
   // grouping of big_tile_of_block
   const int m = G::WGS * a.max_blocks;
   const dim3 grid(ntiles, ntiles % 8 == 0 ? (m + 31) / 32 * 32 : m);
-  if (gateup) hipLaunchKernelGGL((moe_gemm_big_kernel<AFMT, HALF, true>), grid, dim3(G::NT), 0, st, a);
-  else hipLaunchKernelGGL((moe_gemm_big_kernel<AFMT, HALF, false>), grid, dim3(G::NT), 0, st, a);
+  if (gateup) hipLaunchKernelGGL((moe_gemm_big_kernel<AFMT, true>), grid, dim3(G::NT), 0, st, a);
+  else hipLaunchKernelGGL((moe_gemm_big_kernel<AFMT, false>), grid, dim3(G::NT), 0, st, a);
 }
 
 hipError_t launch_moe_gemm_big(const Dsv4GemmArgs& a, bool gateup, hipStream_t st) {
@@ -982,10 +963,7 @@ hipError_t launch_moe_gemm_big(const Dsv4GemmArgs& a, bool gateup, hipStream_t s
     else hipLaunchKernelGGL((moe_gemm_big_bf16_kernel<false>), grid, dim3(CfgBf::NT), 0, st, a);
     return hipGetLastError();
   }
-  // workgroup shape (Cfg): half blocks for E4M3, and for E2M1 while the layer's rows
-  // are too few to fill the CUs with whole blocks
-  if (a.afmt == 0) launch_big<0, true>(a, gateup, ntiles, st);
-  else if (a.R < 32768) launch_big<1, true>(a, gateup, ntiles, st);
-  else launch_big<1, false>(a, gateup, ntiles, st);
+  if (a.afmt == 0) launch_big<0>(a, gateup, ntiles, st);
+  else launch_big<1>(a, gateup, ntiles, st);
   return hipGetLastError();
 }
