@@ -691,6 +691,7 @@ static int layer_forward(int profile, int scale_rule, const void* x, const void*
   }
   if (shared) {  // rows R.. read x row f - R with routing weight 1
     gu.has_shared = 1;
+    gu.shared_blocks = (n_sh + bm - 1) / bm;
     gu.shared_expert = E;
     gu.shared_a_rows = n_sh;
     gu.shared = *shared;
@@ -770,6 +771,7 @@ static int layer_forward(int profile, int scale_rule, const void* x, const void*
   dn.out = (uint16_t*)(base + w.out);
   if (shared) {  // h rows are indexed by flat index for every group
     dn.has_shared = 1;
+    dn.shared_blocks = (n_sh + bm - 1) / bm;
     dn.shared_expert = E;
     dn.shared = *shared;
   }

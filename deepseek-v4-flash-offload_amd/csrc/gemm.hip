@@ -100,7 +100,8 @@ struct AStage<kAfmtBf16> {
 // B operand of one stage: E2M1 weights (16 bytes per lane per MFMA, kNT tiles)
 // or, for the shared expert, E4M3 weights (32 bytes, laid out like the E4M3 A
 // operand). An E4M3 stage holds kNT/2 tiles, so both take the same registers;
-// the E4M3 path covers its kNT tiles in two passes over K.
+// the 64-row kernel covers its kNT tiles in two passes over K and the 16-row one gives
+// them to two workgroups.
 template <bool B8>
 struct BStageT {
   static constexpr int NTB = B8 ? kNT / 2 : kNT;
@@ -350,10 +351,10 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 // tile t for row row0 + r16. Gate/up: hb[t] receives the bf16 h values the SwiGLU produced
 // for intermediate columns col0 + 16 t + 4 g .. + 3 (t = 0, 1), packed in pairs (zero for a
 // padding row), and fr the row's flat index; h is written unless the caller fuses its
-// quantisation.
+// quantisation. Down: the first ntiles tiles are stored.
 template <bool GATEUP, bool SH = false>
 DSV4_DEV void store_tile(const Dsv4GemmArgs& p, const v4f* acc, int row0, int col0, int g, int r16,
-                         uint32_t (*hb)[2] = nullptr, int* fr = nullptr) {
+                         uint32_t (*hb)[2] = nullptr, int* fr = nullptr, int ntiles = kNT) {
   const int f = p.sorted_ids[row0 + r16];
   if (fr) *fr = f;
   if (GATEUP && hb) hb[0][0] = hb[0][1] = hb[1][0] = hb[1][1] = 0u;
@@ -378,13 +379,14 @@ DSV4_DEV void store_tile(const Dsv4GemmArgs& p, const v4f* acc, int row0, int co
   } else {
 #pragma unroll
     for (int t = 0; t < kNT; ++t)
-      *(u32x2_t*)(orow + 16 * t) = u32x2_t{pk_bf16(acc[t][0], acc[t][1]), pk_bf16(acc[t][2], acc[t][3])};
+      if (t < ntiles) *(u32x2_t*)(orow + 16 * t) = u32x2_t{pk_bf16(acc[t][0], acc[t][1]), pk_bf16(acc[t][2], acc[t][3])};
   }
 }
 
 // Gate/up epilogue of one 16-row subtile with the activations as the MFMA's first operand:
-// lane (r16, g) holds rows row0 + 4 g + i (i = 0..3) of column r16 of each tile. Writes h.
-template <bool SH>
+// lane (r16, g) holds rows row0 + 4 g + i (i = 0..3) of column r16 of each of NG gate tiles,
+// then of the NG up tiles. Writes h.
+template <bool SH, int NG>
 DSV4_DEV void store_tile_columns(const Dsv4GemmArgs& p, const v4f* acc, int row0, int col0, int g, int r16) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -393,8 +395,8 @@ DSV4_DEV void store_tile_columns(const Dsv4GemmArgs& p, const v4f* acc, int row0
     uint16_t* orow = p.out + (int64_t)f * p.N + col0 + r16;
     const float w = (!SH || f < p.R - p.shared_a_rows) ? p.topk_w[f] : 1.0f;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const uint32_t gu = pk_bf16(acc[t][i], acc[t + 2][i]);
+    for (int t = 0; t < NG; ++t) {
+      const uint32_t gu = pk_bf16(acc[t][i], acc[t + NG][i]);
       orow[16 * t] = (uint16_t)dsv4::f32_to_bf16(dsv4::swiglu(bf16_lo(gu), bf16_hi(gu), w, p.swiglu_limit));
     }
   }
@@ -433,7 +435,7 @@ DSV4_DEV void quantise_h_mxfp4(const Dsv4GemmArgs& p, const uint32_t (*hb)[2], i
 
 // NTW: the block's routed weights are MFMA-tiled and loaded non-temporally.
 template <int AFMT, bool GATEUP, int NST, bool SH, bool NTW>
-__attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& p, const int mb, const int e) {
+__attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& p, const int mb, const int e, const int half) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // Which operand the weights are (store_tile / store_tile_columns): with the weights
   // first a lane holds 4 columns of one row. A decode block holds one or two routed rows
@@ -462,26 +464,40 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
   BLayout lay{128, 16};  // routed E2M1 weights: checkpoint or MFMA-tiled layout (table pointer bit 0)
   if (GATEUP) {
     col0 = blockIdx.x * (kWaves * 32) + wave * 32;  // 32 intermediate columns: 2 gate + 2 up tiles
+    if (shared) {  // E4M3 rows, twice the bytes: 16 columns per workgroup, one gate and one up tile
+      col0 += 16 * half;
+      const int64_t row = col0 + r16;
+      bt[0] = ex.w1p + row * brow_bytes;
+      bt[1] = ex.w3p + row * brow_bytes;
+      bst[0] = ex.w1s + row * bsrow;
+      bst[1] = ex.w3s + row * bsrow;
+    } else {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int64_t row = col0 + 16 * t + r16;
-      if (shared) {  // E4M3 rows, checkpoint layout (the E4M3 loads add their own offsets)
-        bt[t] = ex.w1p + row * brow_bytes;
-        bt[t + 2] = ex.w3p + row * brow_bytes;
-      } else {  // w1 and w3 of an expert share one layout
+      for (int t = 0; t < 2; ++t) {  // w1 and w3 of an expert share one layout
+        const int64_t row = col0 + 16 * t + r16;
         bt[t] = b_lane_base<NTW>(ex.w1p, row, brow_bytes, NST, lane, lay);
         bt[t + 2] = b_lane_base<NTW>(ex.w3p, row, brow_bytes, NST, lane, lay);
+        bst[t] = ex.w1s + row * bsrow;
+        bst[t + 2] = ex.w3s + row * bsrow;
       }
-      bst[t] = ex.w1s + row * bsrow;
-      bst[t + 2] = ex.w3s + row * bsrow;
     }
   } else {
     col0 = blockIdx.x * (kWaves * 64) + wave * 64;
+    if (shared) {  // two tiles per workgroup
+      col0 += 32 * half;
 #pragma unroll
-    for (int t = 0; t < kNT; ++t) {
-      const int64_t row = col0 + 16 * t + r16;
-      bt[t] = shared ? ex.w2p + row * brow_bytes : b_lane_base<NTW>(ex.w2p, row, brow_bytes, NST, lane, lay);
-      bst[t] = ex.w2s + row * bsrow;
+      for (int t = 0; t < kNT / 2; ++t) {
+        const int64_t row = col0 + 16 * t + r16;
+        bt[t] = ex.w2p + row * brow_bytes;
+        bst[t] = ex.w2s + row * bsrow;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < kNT; ++t) {
+        const int64_t row = col0 + 16 * t + r16;
+        bt[t] = b_lane_base<NTW>(ex.w2p, row, brow_bytes, NST, lane, lay);
+        bst[t] = ex.w2s + row * bsrow;
+      }
     }
   }
 
@@ -493,18 +509,16 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
   // DSV4_GEMM_PREFETCH = P > 0 the loads of stage j+P are issued before the
   // MFMAs of stage j and a scheduling barrier keeps them there (a P+1 deep
   // register ring); with P = 0 the compiler schedules freely.
-  // T0: first tile of this pass (E4M3 weights: two passes of kNT/2 tiles).
   // NT: non-temporal weight loads (MFMA-tiled routed weights only: on the
   // checkpoint layout they measured 9% slower than plain loads).
-  auto kloop = [&](auto b8, auto t0c, auto ntc) {
+  auto kloop = [&](auto b8, auto ntc) {
     constexpr bool B8 = decltype(b8)::value;
-    constexpr int t0 = decltype(t0c)::value;
     constexpr bool NT = decltype(ntc)::value;
     constexpr int NTB = BStageT<B8>::NTB;
     constexpr int P = DSV4_GEMM_PREFETCH;
     constexpr int RING = P + 1;
-    const uint8_t* const* btp = bt + t0;
-    const uint8_t* const* bstp = bst + t0;
+    const uint8_t* const* btp = bt;
+    const uint8_t* const* bstp = bst;
     AStage<AFMT> a[RING];
     BStageT<B8> b[RING];
     RowScales<NST> as_row, bs_row[NTB];
@@ -526,10 +540,10 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
 #pragma unroll
       for (int t = 0; t < NTB; ++t) b[j % RING].s[t] = stage_scales<NST>(bs_row[t], j, r16, g);
       if constexpr (AFMT == kAfmtBf16) {
-        compute_bf16<B8, kWRows>(acc + t0, a[j % RING], b[j % RING]);
+        compute_bf16<B8, kWRows>(acc, a[j % RING], b[j % RING]);
       } else {
         a[j % RING].s = stage_scales<NST>(as_row, j, r16, g);
-        compute<AFMT, B8, kWRows>(acc + t0, a[j % RING], b[j % RING]);
+        compute<AFMT, B8, kWRows>(acc, a[j % RING], b[j % RING]);
       }
       if constexpr (P > 0) __builtin_amdgcn_sched_barrier(0);
     }
@@ -538,12 +552,11 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
   // the loads' immediate-offset range) they led it to keep a 64-bit address
   // per stage live, +20 VGPRs in the down GEMM.
   if constexpr (NTW) asm volatile("" : "+s"(lay.stage_stride), "+s"(lay.mfma_stride));
-  auto routed = [&] { kloop(std::false_type{}, std::integral_constant<int, 0>{}, std::integral_constant<bool, NTW>{}); };
+  auto routed = [&] { kloop(std::false_type{}, std::integral_constant<bool, NTW>{}); };
   if (have_w) {
     if constexpr (AFMT == 0 && SH) {  // E4M3 weights only meet E4M3 activations (bf16 profile)
       if (shared) {
-        kloop(std::true_type{}, std::integral_constant<int, 0>{}, std::false_type{});
-        kloop(std::true_type{}, std::integral_constant<int, kNT / 2>{}, std::false_type{});
+        kloop(std::true_type{}, std::false_type{});
       } else {
         routed();
       }
@@ -558,9 +571,10 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
     store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, hb, &f);
     quantise_h_mxfp4(p, hb, f, col0, g);
   } else if constexpr (kWRows) {
-    store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16);
+    store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, nullptr, nullptr, shared ? kNT / 2 : kNT);
   } else {
-    store_tile_columns<SH>(p, acc, mb * kBM, col0, g, r16);
+    if (shared) store_tile_columns<SH, 1>(p, acc, mb * kBM, col0, g, r16);
+    else store_tile_columns<SH, 2>(p, acc, mb * kBM, col0, g, r16);
   }
 }
 
@@ -571,14 +585,22 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
 // the register count by up to 100 VGPRs).
 template <int AFMT, bool GATEUP, int NST, bool SH>
 __global__ __launch_bounds__(64 * kWaves) void moe_gemm_kernel(Dsv4GemmArgs p) {
-  const int mb = blockIdx.y;
+  // The shared expert's blocks lead the layout and run as two workgroups per 32 (gate/up) or
+  // 64 (down) columns: its E4M3 rows are twice as long as a routed expert's, and one
+  // workgroup that took the tiles in two passes over K was the launch's tail at small
+  // batches (one token, top-6: gate/up 18.0 -> 14.4 us, down 10.9 -> 8.9).
+  int mb = blockIdx.y, half = 0;
+  if (SH) {
+    if (mb < 2 * p.shared_blocks) half = mb & 1, mb >>= 1;
+    else mb -= p.shared_blocks;
+  }
   if (mb * kBM >= p.num_post_padded[0]) return;
   const int e = p.block_expert[mb];
   const bool shared = SH && e == p.shared_expert;
   if (kNtLoads && !shared && tiled_ptr(GATEUP ? p.experts[e].w1p : p.experts[e].w2p))
-    moe_gemm_block<AFMT, GATEUP, NST, SH, true>(p, mb, e);
+    moe_gemm_block<AFMT, GATEUP, NST, SH, true>(p, mb, e, half);
   else
-    moe_gemm_block<AFMT, GATEUP, NST, SH, false>(p, mb, e);
+    moe_gemm_block<AFMT, GATEUP, NST, SH, false>(p, mb, e, half);
 }
 
 // ---------------------------------------------------------------------------
@@ -1016,7 +1038,7 @@ template <bool GATEUP, int NST, bool SH>
 static void launch_nst_sh(const Dsv4GemmArgs& a, hipStream_t st) {
   const int cols_per_wave = GATEUP ? 32 : 64;
   if (a.block_m == kBM) {  // decode-shaped: single-wave workgroups
-    const dim3 grid(a.N / (kWaves * cols_per_wave), a.max_blocks);
+    const dim3 grid(a.N / (kWaves * cols_per_wave), a.max_blocks + (SH ? a.shared_blocks : 0));
     if constexpr (!SH) {  // bf16 activations: routed experts only
       if (a.afmt == kAfmtBf16) {
         hipLaunchKernelGGL((moe_gemm_kernel<kAfmtBf16, GATEUP, NST, false>), grid, dim3(64 * kWaves), 0, st, a);
