@@ -105,6 +105,12 @@ def test_route_matches_oracle(gpu, T, D, E, K, scoring, use_bias, renorm, xdtype
     _check(out_w.cpu().numpy(), out_ids.cpu().numpy(), ref_w, ref_ids, sc, bias, K)
 
 
+@pytest.mark.parametrize("T,D,xdtype", [(8193, 2048, "bf16"), (8200, 1536, "fp32"), (16400, 1024, "bf16")])
+def test_route_several_k_chunks_per_workgroup(gpu, T, D, xdtype):
+    """Token counts that split K in fewer than D / 512 parts: workgroups walk 2 or 3 chunks."""
+    test_route_matches_oracle(gpu, T, D, 256, 6, "sqrtsoftplus", True, True, xdtype)
+
+
 @pytest.mark.parametrize("tab_dtype", [torch.int32, torch.int64])
 def test_route_hash_layer_and_bad_ids(gpu, tab_dtype):
     T, D, E, K, V = 12, 4096, 256, 6, 1000
