@@ -346,6 +346,9 @@ DSV4_DEV float group_max(float v) {
 }
 
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+// as stored to a caller's h / out, which need only be aligned to its 2-byte elements: still
+// one global_store_dwordx2 (the amdhsa ABI runs in unaligned access mode)
+typedef u32x2_t u32x2_out __attribute__((aligned(2)));
 
 // Epilogue of one 16-row subtile: lane (r16, g) holds columns 16 t + 4 g + i (i = 0..3) of
 // tile t for row row0 + r16. Gate/up: hb[t] receives the bf16 h values the SwiGLU produced
@@ -374,12 +377,12 @@ DSV4_DEV void store_tile(const Dsv4GemmArgs& p, const v4f* acc, int row0, int co
                              dsv4::swiglu(bf16_lo(gu1), bf16_hi(gu1), w, p.swiglu_limit));
         if (hb) hb[t][i >> 1] = h2[i >> 1];
       }
-      if (!p.hq_skip_h) *(u32x2_t*)(orow + 16 * t) = u32x2_t{h2[0], h2[1]};
+      if (!p.hq_skip_h) *(u32x2_out*)(orow + 16 * t) = u32x2_t{h2[0], h2[1]};
     }
   } else {
 #pragma unroll
     for (int t = 0; t < kNT; ++t)
-      if (t < ntiles) *(u32x2_t*)(orow + 16 * t) = u32x2_t{pk_bf16(acc[t][0], acc[t][1]), pk_bf16(acc[t][2], acc[t][3])};
+      if (t < ntiles) *(u32x2_out*)(orow + 16 * t) = u32x2_t{pk_bf16(acc[t][0], acc[t][1]), pk_bf16(acc[t][2], acc[t][3])};
   }
 }
 

@@ -367,7 +367,9 @@ DSV4_DEV void wave_lds_fence() {
 // f) to base + f * row_stride; rows with f >= R (padding) are left out.
 // Non-temporal: the outputs of the sizes this kernel serves do not stay in the L2 until
 // their reader runs, and leave it to the operands (layer at 16384 tokens 3278 -> 3252 us
-// a4w4, 3812 -> 3800 us bf16; 2048 tokens unchanged).
+// a4w4, 3812 -> 3800 us bf16; 2048 tokens unchanged). base need only be aligned to 2 bytes
+// (a caller's h): still one global_store_dwordx4, the amdhsa ABI runs in unaligned access mode.
+typedef v4i v4i_out __attribute__((aligned(2)));
 template <int ROWB>
 DSV4_DEV void store_staged_rows(const uint8_t* st, int lane, int fr, int R, uint8_t* base, int64_t row_stride) {
   constexpr int CPR = ROWB / 16;        // 16-byte pieces per row
@@ -380,7 +382,7 @@ DSV4_DEV void store_staged_rows(const uint8_t* st, int lane, int fr, int R, uint
     const int row = it * RPI + lane / CPR, ch = lane % CPR;
     const int f = __shfl(fr, row, 64);
     const v4i v = *(const v4i*)(st + row * stage_pitch<ROWB>() + 16 * ch);
-    if (f < R) __builtin_nontemporal_store(v, (v4i*)(base + (int64_t)f * row_stride + 16 * ch));
+    if (f < R) __builtin_nontemporal_store(v, (v4i_out*)(base + (int64_t)f * row_stride + 16 * ch));
   }
   wave_lds_fence();
 }

@@ -216,7 +216,8 @@ int dsv4_moe_combine(const void* out_flat, const void* topk_ids, int ids_int64, 
  * tiles) or 256 (large-tile workgroups: 32x32x64 scaled MFMAs for E4M3/E2M1
  * A, 32x32x16 bf16 MFMAs on weights dequantised in registers for bf16 A; D a
  * multiple of 1024 for gate/up, I of 1024 and D of 256 for down); D and I must
- * be 256 * 2^n (512..4096) and I a multiple of 128. */
+ * be 256 * 2^n (512..4096) and I a multiple of 128. a must be 16-byte aligned,
+ * a_scale 4, h_out 2 (its elements). */
 int dsv4_moe_gemm_gateup(int afmt, const void* a, const void* a_scale, int a_row_div, const int32_t* sorted_ids,
                          const int32_t* block_expert, const int32_t* num_post_padded, int R, int block_m,
                          int max_blocks, const void* expert_table, int D, int I, const float* topk_w,
@@ -224,7 +225,8 @@ int dsv4_moe_gemm_gateup(int afmt, const void* a, const void* a_scale, int a_row
 
 /* Grouped down GEMM: out[f] = bf16(a[f] @ W2[e]^T) for every routed row.
  * Replaces npu_grouped_matmul of deepseek_v4.py:190-193 / 241.
- * a: [R, I] (E4M3) or [R, I/2] (E2M1) by flat index, a_scale [R, I/32]. */
+ * a: [R, I] (E4M3) or [R, I/2] (E2M1) by flat index, a_scale [R, I/32]. out must
+ * be 2-byte aligned (its elements), with block_m 256 16-byte aligned. */
 int dsv4_moe_gemm_down(int afmt, const void* a, const void* a_scale, const int32_t* sorted_ids,
                        const int32_t* block_expert, const int32_t* num_post_padded, int R, int block_m,
                        int max_blocks, const void* expert_table, int I, int D, void* out, void* stream);

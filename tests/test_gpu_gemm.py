@@ -22,7 +22,7 @@ import torch
 from oracle import mxfp4 as Q
 from oracle import moe as M
 from _parity import check_bound, elementwise_rel, gemm_bound, swiglu_bound
-from dsv4_hip import (ops, synth, AFMT_E2M1, AFMT_E4M3, PROFILE_A4W4, PROFILE_BF16, PROFILE_BF16_PURE,
+from dsv4_hip import (ops, synth, AFMT_BF16, AFMT_E2M1, AFMT_E4M3, PROFILE_A4W4, PROFILE_BF16, PROFILE_BF16_PURE,
                       RULE_OCP_FLOOR, RULE_CEIL_DIV6)
 
 pytestmark = pytest.mark.gpu
@@ -153,6 +153,53 @@ def _stage_case(gpu, profile, T, K, E, D, I, bm):
         assert np.array_equal(out_gpu, out_want), "a4w4 down: not bit-exact"
     else:
         check_bound(out_gpu, out_want, gemm_bound(out_want, out_abs), f"down {profile} bm={bm}")
+
+
+@pytest.mark.parametrize("afmt,bm", [(AFMT_E4M3, 16), (AFMT_E4M3, 64), (AFMT_E4M3, 128), (AFMT_E4M3, 256),
+                                     (AFMT_E2M1, 16), (AFMT_E2M1, 64), (AFMT_E2M1, 128), (AFMT_E2M1, 256),
+                                     (AFMT_BF16, 16), (AFMT_BF16, 64), (AFMT_BF16, 256)])
+@pytest.mark.parametrize("shift", [1, 3, 4])
+def test_grouped_gemm_outputs_need_element_alignment_only(gpu, afmt, bm, shift):
+    """h_out and out `shift` elements past an aligned address (2, 6 and 8 bytes): the same bits as
+    aligned ones, and nothing written around them. (out of 256-row blocks must be 16-byte aligned.)"""
+    T, K, E, D, I = 37, 4, 4, 1024, 1024
+    ids, w, xb, host, devw, table = _case(T, K, E, D, I, 5, gpu)
+    al = ops.moe_align(_dev(ids, gpu), _dev(w, gpu), E, bm)
+    g = torch.Generator(device=gpu).manual_seed(bm)
+
+    def operand(rows, cols):
+        if afmt == AFMT_BF16:
+            return torch.randn(rows, cols, generator=g, device=gpu).to(torch.bfloat16), None
+        a = torch.randn(rows, cols, generator=g, device=gpu).to(torch.bfloat16)
+        if afmt == AFMT_E2M1:
+            packed, scale, _ = ops.mxfp4_act_quant(a, RULE_OCP_FLOOR)
+            return packed, scale
+        q = ops.fp8_act_quant(a, 128, want_codes=True, want_e8m0x4=True)
+        return q["codes"], q["e8m0x4"]
+
+    def shifted(rows, cols):
+        buf = torch.full((rows * cols + 16,), 7.0, dtype=torch.bfloat16, device=gpu)
+        return buf, buf[shift:shift + rows * cols].view(rows, cols)
+
+    a, a_s = operand(T, D)
+    wf = _dev(w.reshape(-1), gpu)
+    want = ops.gemm_gateup(afmt, a, a_s, K, al, table, D, I, wf, 10.0)
+    buf, h = shifted(T * K, I)
+    ops.gemm_gateup(afmt, a, a_s, K, al, table, D, I, wf, 10.0, out=h)
+    torch.cuda.synchronize()
+    assert torch.equal(h.view(torch.int16), want.view(torch.int16))
+    assert (buf[:shift] == 7.0).all() and (buf[shift + h.numel():] == 7.0).all()
+    a, a_s = operand(T * K, I)
+    want = ops.gemm_down(afmt, a, a_s, al, table, I, D)
+    buf, out = shifted(T * K, D)
+    if bm == 256:
+        with pytest.raises(ops._lib.Dsv4Error, match="16-byte aligned output"):
+            ops.gemm_down(afmt, a, a_s, al, table, I, D, out=out)
+        return
+    ops.gemm_down(afmt, a, a_s, al, table, I, D, out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert (buf[:shift] == 7.0).all() and (buf[shift + out.numel():] == 7.0).all()
 
 
 def test_grouped_gemm_empty_group_pattern(gpu):
