@@ -328,14 +328,9 @@ DSV4_DEV int64_t a_row(const Dsv4GemmArgs& p, int f) {
   return f < r0 ? (int64_t)(f / p.a_row_div) : (f < p.R ? (int64_t)(f - r0) : 0);
 }
 
-// two floats -> packed bf16 (RNE, NaN -> 0x7fc0 as f32_to_bf16), low half = a
-DSV4_DEV uint32_t pk_bf16(float a, float b) {
-  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-  const uint32_t w = __builtin_bit_cast(uint32_t, v2bf{(__bf16)a, (__bf16)b});
-  return (a != a ? 0x7fc0u : w & 0xffffu) | (b != b ? 0x7fc00000u : w & 0xffff0000u);
-}
-DSV4_DEV float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-DSV4_DEV float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+using dsv4::bf16_hi;
+using dsv4::bf16_lo;
+using dsv4::pk_bf16;
 
 // maximum of a value over the four lane groups g (lanes r, r + 16, r + 32, r + 48)
 DSV4_DEV float group_max(float v) {

@@ -286,41 +286,21 @@ DSV4_DEV void big_mfma(typename Big<AFMT>::Acc& acc, const BigFrag<AFMT>& F, con
 // 8q + 4(l/32) + e of every 32-column weight tile): SwiGLU, the quantisation blocks'
 // maxima (in-lane, then across the lane pair l, l ^ 32, then - FP8 h only - across the
 // WN waves of a token row through the LDS) and the packing all stay in registers.
-// bf16 / E4M3 / E2M1 conversions use the gfx950 converters, which agree bit for bit
-// with the library's software quantisers on every input they see here (RNE; E4M3 after
-// the clamp to +-448; E2M1 with the sign of the input, whose -0 the rule-0 path
-// turns into +0 as that rule wants).
+// The bf16 / E4M3 / E2M1 conversions are those of the 16/64-row kernels and the stand-alone
+// quantisers (quant_dev.h), so a row gets the same codes whichever kernel its expert runs
+// on, non-finite values included. pk_bf16's NaN selects, six VALU instructions per pair,
+// cost the 16384-token layer 1 % here (3476 -> 3511 us, bf16): the packing is the bare
+// converter, the block maxima carry NaN, and a wave that finds one there repairs its h.
+// (A NaN of the down outputs keeps its sign and payload; the combine does not.)
+using dsv4::bf16_hi;
+using dsv4::bf16_lo;
+using dsv4::cvt_pk_bf16;
+using dsv4::pk_bf16;
 
 // max of x over the lane pair (l, l ^ 32)
 DSV4_DEV float max_pair(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
   return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
-}
-
-// two floats -> packed bf16 (RNE), low half = a
-DSV4_DEV uint32_t pk_bf16(float a, float b) {
-  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-  const v2bf v = v2bf{(__bf16)a, (__bf16)b};
-  return __builtin_bit_cast(uint32_t, v);
-}
-DSV4_DEV float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-DSV4_DEV float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-
-// 4 E4M3 codes of a * inv .. d * inv (inv = 2^-k), byte 0 = a
-DSV4_DEV uint32_t pk_fp8x4(float a, float b, float c, float d, float inv) {
-  const float m = 448.0f;
-  const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(fmaxf(a * inv, -m), m), fminf(fmaxf(b * inv, -m), m), 0, false);
-  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(fminf(fmaxf(c * inv, -m), m), fminf(fmaxf(d * inv, -m), m), lo, true);
-}
-
-// E2M1 nibble pair of a * inv, b * inv (low nibble = a) under scale rule `rule`
-DSV4_DEV uint32_t pk_fp4x2(float a, float b, float inv, int rule) {
-  float ya = fminf(fmaxf(a * inv, -6.0f), 6.0f), yb = fminf(fmaxf(b * inv, -6.0f), 6.0f);
-  if (rule == 0) {  // the sign of a value that is exactly zero is +
-    ya = ya == 0.0f ? 0.0f : ya;
-    yb = yb == 0.0f ? 0.0f : yb;
-  }
-  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, ya, yb, 1.0f, 0) & 0xffu;
 }
 
 // Block -> tile mapping. Workgroups are dispatched to the 8 XCDs round-robin by
@@ -408,6 +388,7 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
     // h for columns cw + 32 h + 8 q + 4 g2 + e of token tile tt, packed bf16 pairs
     uint32_t hp[G::TT][H][4][2];
     float rmax[G::TT][H];  // per 32-column block, this lane's half of it
+    bool nan = false;
 #pragma unroll
     for (int tt = 0; tt < G::TT; ++tt)
 #pragma unroll
@@ -419,15 +400,33 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
           for (int e = 0; e < 4; e += 2) {
             const int r = 4 * q + e;
             // gate (tile h) and up (tile H + h) of the same column, rounded to bf16
-            const uint32_t gu0 = pk_bf16(acc[tt][h][r], acc[tt][H + h][r]);
-            const uint32_t gu1 = pk_bf16(acc[tt][h][r + 1], acc[tt][H + h][r + 1]);
-            const uint32_t hw = pk_bf16(dsv4::swiglu(bf16_lo(gu0), bf16_hi(gu0), wr[tt], p.swiglu_limit),
-                                        dsv4::swiglu(bf16_lo(gu1), bf16_hi(gu1), wr[tt], p.swiglu_limit));
+            const uint32_t gu0 = cvt_pk_bf16(acc[tt][h][r], acc[tt][H + h][r]);
+            const uint32_t gu1 = cvt_pk_bf16(acc[tt][h][r + 1], acc[tt][H + h][r + 1]);
+            const float h0 = dsv4::swiglu(bf16_lo(gu0), bf16_hi(gu0), wr[tt], p.swiglu_limit);
+            const float h1 = dsv4::swiglu(bf16_lo(gu1), bf16_hi(gu1), wr[tt], p.swiglu_limit);
+            const uint32_t hw = cvt_pk_bf16(h0, h1);
             hp[tt][h][q][e >> 1] = hw;
-            m = fmaxf(m, fmaxf(fabsf(bf16_lo(hw)), fabsf(bf16_hi(hw))));
+            m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(bf16_lo(hw))), fabsf(bf16_hi(hw)));
           }
         rmax[tt][h] = m;
+        nan |= m != m;
       }
+    const bool wave_nan = __builtin_expect(__ballot(nan) != 0, 0);
+    if (wave_nan) {  // canonical NaN, and maxima that leave it out
+#pragma unroll
+      for (int tt = 0; tt < G::TT; ++tt)
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          float m = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            uint32_t& w = hp[tt][h][i >> 1][i & 1];
+            w = pk_bf16(bf16_lo(w), bf16_hi(w));
+            m = fmaxf(m, fmaxf(fabsf(bf16_lo(w)), fabsf(bf16_hi(w))));
+          }
+          rmax[tt][h] = m;
+        }
+    }
     if (!p.hq_skip_h && p.out) {
 #pragma unroll
       for (int tt = 0; tt < G::TT; ++tt) {
@@ -441,6 +440,17 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
       }
     }
     if (p.hq_mode == 2) {  // MXFP4 h: one 32-column block per (tt, h), half of it in each lane of a pair
+      if (wave_nan) {  // infinity in its place clamps to the code mxfp4_clamped gives NaN
+        const uint32_t inf = p.hq_rule == 0 ? 0xff80u : 0x7f80u;
+        auto num = [&](uint32_t b) { return b == 0x7fc0u ? inf : b; };
+#pragma unroll
+        for (int tt = 0; tt < G::TT; ++tt)
+#pragma unroll
+          for (int i = 0; i < 8 * H; ++i) {
+            uint32_t& w = hp[tt][i >> 3][(i >> 1) & 3][i & 1];
+            w = num(w & 0xffffu) | num(w >> 16) << 16;
+          }
+      }
 #pragma unroll
       for (int tt = 0; tt < G::TT; ++tt) {
 #pragma unroll
@@ -450,8 +460,9 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
-            const uint32_t nib = pk_fp4x2(bf16_lo(w0), bf16_hi(w0), inv, p.hq_rule) |
-                                 pk_fp4x2(bf16_lo(w1), bf16_hi(w1), inv, p.hq_rule) << 8;
+            auto y = [&](float v) { return dsv4::mxfp4_clamped_number(v, inv, p.hq_rule); };
+            const uint32_t nib = dsv4::e2m1_pair<1>(dsv4::e2m1_pair<0>(0u, y(bf16_lo(w0)), y(bf16_hi(w0))),
+                                                    y(bf16_lo(w1)), y(bf16_hi(w1)));
             *(uint16_t*)(st + r32 * stage_pitch<16 * H>() + 16 * h + 4 * q + 2 * g2) = (uint16_t)nib;
           }
           if (g2 == 0 && fr[tt] < p.R) p.hq_scale[(int64_t)fr[tt] * (p.N / 32) + cw / 32 + h] = (uint8_t)(k + 127);
@@ -486,8 +497,8 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const uint32_t w0 = hp[tt][h][q][0], w1 = hp[tt][h][q][1];
-            *(uint32_t*)(st + r32 * stage_pitch<32 * H>() + 32 * h + 8 * q + 4 * g2) =
-                pk_fp8x4(bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1), inv);
+            const float y[4] = {bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1)};
+            *(uint32_t*)(st + r32 * stage_pitch<32 * H>() + 32 * h + 8 * q + 4 * g2) = dsv4::fp8_codes4(y, inv);
           }
         store_staged_rows<32 * H>(st, lane, fr[tt], p.R, p.hq_codes + cw, p.N);
         if (wn == 0 && g2 == 0 && fr[tt] < p.R)  // the block's four scale bytes (N, c0: multiples of 128)
@@ -503,8 +514,8 @@ DSV4_DEV void big_epilogue(const Dsv4GemmArgs& p, v16f (&acc)[G::TT][G::WT], uin
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int r = 4 * q;
-          *(v2u*)(st + r32 * stage_pitch<64 * G::WT>() + 64 * wt + 16 * q + 8 * g2) =
-              v2u{pk_bf16(acc[tt][wt][r], acc[tt][wt][r + 1]), pk_bf16(acc[tt][wt][r + 2], acc[tt][wt][r + 3])};
+          *(v2u*)(st + r32 * stage_pitch<64 * G::WT>() + 64 * wt + 16 * q + 8 * g2) = v2u{
+              cvt_pk_bf16(acc[tt][wt][r], acc[tt][wt][r + 1]), cvt_pk_bf16(acc[tt][wt][r + 2], acc[tt][wt][r + 3])};
         }
       store_staged_rows<64 * G::WT>(st, lane, fr[tt], p.R, (uint8_t*)(p.out + cw), 2 * (int64_t)p.N);
     }

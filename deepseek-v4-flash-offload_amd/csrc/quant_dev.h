@@ -10,6 +10,19 @@
 
 namespace dsv4 {
 
+// two floats -> packed bf16 (RNE, NaN -> 0x7fc0 as f32_to_bf16), low half = a;
+// cvt_pk_bf16: the converter alone, which keeps a NaN's sign and payload
+DSV4_DEV uint32_t cvt_pk_bf16(float a, float b) {
+  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, v2bf{(__bf16)a, (__bf16)b});
+}
+DSV4_DEV uint32_t pk_bf16(float a, float b) {
+  const uint32_t w = cvt_pk_bf16(a, b);
+  return (a != a ? 0x7fc0u : w & 0xffffu) | (b != b ? 0x7fc00000u : w & 0xffff0000u);
+}
+DSV4_DEV float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
+DSV4_DEV float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+
 // silu(min(g, L)) * clamp(u, +-L) * w for bf16-rounded g, u (deepseek_v4.py:184-187),
 // the one formula of every gate/up epilogue: a token row gets the same h whichever
 // kernel its expert runs on. limit <= 0: no clamps.
@@ -140,6 +153,11 @@ DSV4_DEV uint32_t e2m1_pair(uint32_t old, float a, float b) {
 DSV4_DEV float mxfp4_clamped(float f, float inv, int rule) {
   if (rule == 0) return fminf(fmaxf(f * inv, -6.0f), 6.0f) + 0.0f;  // -0 + 0 = +0
   return copysignf(fminf(fabsf(f * inv), 6.0f), f);
+}
+// the same for f that is not NaN, one instruction shorter under rule 1
+DSV4_DEV float mxfp4_clamped_number(float f, float inv, int rule) {
+  const float y = fminf(fmaxf(f * inv, -6.0f), 6.0f);
+  return rule == 0 ? y + 0.0f : y;
 }
 
 // Group g (already loaded: v) of a tensor; `live` must be the same for the 4 lanes of a block.

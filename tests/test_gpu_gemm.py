@@ -202,6 +202,61 @@ def test_grouped_gemm_outputs_need_element_alignment_only(gpu, afmt, bm, shift):
     assert (buf[:shift] == 7.0).all() and (buf[shift + out.numel():] == 7.0).all()
 
 
+@pytest.mark.parametrize("profile,rule", [("a4w4", RULE_OCP_FLOOR), ("a4w4", RULE_CEIL_DIV6),
+                                          ("bf16", RULE_OCP_FLOOR), ("bf16_pure", RULE_OCP_FLOOR)])
+def test_nan_rows_agree_between_kernels(gpu, profile, rule):
+    """Weight scale bytes of 255 and no clamps: h and column 5 of the outputs hold NaN. Eight tokens'
+    rows on an expert in 64-row blocks and the same rows on one in 256-row blocks (same weights) give
+    the same h bits, and the same layer outputs: a4w4 bit for bit (its sums are exact), bf16 within
+    the summation order of the E4M3 products (rel 1e-2, as the parity tests), pure bf16 NaN alike."""
+    T, K, E, D, I, n = 8192 if profile == "bf16_pure" else 2048, 8, 16, 1024, 1024, 8
+    host = synth.expert_weights(3, D, I)
+    for row, block in ((0, 1), (37, 0), (I - 1, D // 32 - 1)):
+        host["w1s"][row, block] = 255
+    host["w3s"][100, 2] = 255
+    host["w2s"][5, 3] = 255
+    dev = {k: _dev(v, gpu) for k, v in host.items()}
+    table = ops.expert_table({e: dev for e in range(E)}, E, gpu)
+    ids = torch.zeros((T, K), dtype=torch.int32, device=gpu)      # expert 0: every row but
+    ids[:n] = 15                                                  # the first n tokens' (64 rows)
+    x = torch.randn(T, D, generator=torch.Generator(device=gpu).manual_seed(2), device=gpu).to(torch.bfloat16)
+    x[n:2 * n] = x[:n]
+    w = torch.rand(T, K, generator=torch.Generator(device=gpu).manual_seed(3), device=gpu)
+    w[n:2 * n] = w[:n]
+
+    def operand(v):
+        if profile == "a4w4":
+            return AFMT_E2M1, *ops.mxfp4_act_quant(v, rule)[:2]
+        if profile == "bf16_pure":
+            return AFMT_BF16, v, None
+        q = ops.fp8_act_quant(v, 128, want_codes=True, want_e8m0x4=True)
+        return AFMT_E4M3, q["codes"], q["e8m0x4"]
+
+    al = {bm: ops.moe_align(ids, w, E, bm) for bm in (16, 64, 256)}
+    afmt, a, a_s = operand(x)
+    h = {bm: ops.gemm_gateup(afmt, a, a_s, K, al[bm], table, D, I, w.view(-1), 0.0) for bm in al}
+    afmt, a, a_s = operand(x.repeat_interleave(K, 0)[:, :I].contiguous())
+    out = {bm: ops.gemm_down(afmt, a, a_s, al[bm], table, I, D) for bm in al}
+    y = ops.LayerRunner(gpu, E, D, I).forward(
+        x, ids, w, table, profile={"bf16": PROFILE_BF16, "a4w4": PROFILE_A4W4, "bf16_pure": PROFILE_BF16_PURE}[profile],
+        rule=rule, swiglu_limit=0.0)
+    torch.cuda.synchronize()
+    for bm in h:
+        nan = torch.isnan(h[bm])
+        assert nan[:, [0, 37, I - 1, 100]].all() and int(nan.sum()) == 4 * T * K
+        assert (h[bm][nan].view(torch.int16) == 0x7fc0).all(), bm
+        assert torch.isnan(out[bm][:, 5]).all() and int(torch.isnan(out[bm]).sum()) == T * K, bm
+    y = y.float()
+    assert torch.isnan(y[:, 5]).all()
+    y = torch.cat((y[:, :5], y[:, 6:]), 1)
+    if profile == "a4w4":
+        assert torch.isfinite(y).all() and torch.equal(y[:n], y[n:2 * n])
+    elif profile == "bf16":
+        assert torch.isfinite(y).all() and (y[:n] - y[n:2 * n]).abs().max() <= 1e-2 * y[:n].abs().max()
+    else:
+        assert torch.isnan(y[:2 * n]).all()
+
+
 def test_grouped_gemm_empty_group_pattern(gpu):
     # _bench_gmm.py:8-22: groups [2, 0, 3] -> expert 1 receives no rows
     E, D, I, K = 3, 512, 512, 1
