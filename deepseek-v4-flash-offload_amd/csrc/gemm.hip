@@ -1094,6 +1094,11 @@ static hipError_t launch(const Dsv4GemmArgs& a, hipStream_t st) {
   if (a.block_m != 16 && a.block_m != 64 && a.block_m != 128) return hipErrorInvalidValue;
   // bf16 activations: 16- or 64-row blocks, without a shared expert or a fused h quantisation
   if (a.afmt == kAfmtBf16 && (a.block_m == 128 || a.has_shared || (GATEUP && a.hq_mode))) return hipErrorInvalidValue;
+  // the 16-row gate/up quantises h only to MXFP4 and only with E2M1 activations (a wave holds no
+  // whole FP8 block; the E4M3 and bf16 forms always write h), and needs the shared blocks' count
+  if (a.block_m == kBM && GATEUP && (a.hq_mode || a.hq_skip_h) && !(a.afmt == 1 && a.hq_mode == 2))
+    return hipErrorInvalidValue;
+  if (a.block_m == kBM && a.has_shared && a.shared_blocks <= 0) return hipErrorInvalidValue;
   switch (a.Kdim / kStageK) {
     case 2: launch_nst<GATEUP, 2>(a, st); break;
     case 4: launch_nst<GATEUP, 4>(a, st); break;

@@ -4,6 +4,7 @@ declares, and rejects bad arguments on the host before touching a GPU."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -129,6 +130,39 @@ def test_gemm_and_layer_validation():
     rc, msg = _err(lib.dsv4_moe_layer_forward(0, 1, None, None, 1, None, 8, 8, 256, 4096, 2048, None,
                                               ctypes.c_float(10.0), None, 0, None, None))
     assert rc == -1
+
+
+def test_gemm_launch_refuses_options_its_kernel_lacks(tmp_path):
+    """The internal launchers answer hipErrorInvalidValue, before any launch, for epilogue options the
+    16-row gate/up does not have: h quantisation (or leaving h out) with E4M3 or bf16 activations,
+    FP8 h at all, and shared-expert rows without the number of their blocks."""
+    src = tmp_path / "t.cpp"
+    src.write_text(r"""
+#include <cstdio>
+#include <initializer_list>
+#include "kernels.h"
+int main() {
+  auto rc = [](int afmt, int hq_mode, int skip, int shared, int shared_blocks) {
+    Dsv4GemmArgs g{};
+    g.afmt = afmt, g.block_m = 16, g.max_blocks = 1, g.R = 16, g.Kdim = 512, g.N = 512, g.a_row_div = 1;
+    g.hq_mode = hq_mode, g.hq_skip_h = skip, g.has_shared = shared, g.shared_blocks = shared_blocks;
+    return (int)launch_moe_gemm_gateup(g, nullptr);
+  };
+  std::printf("%d", (int)hipErrorInvalidValue);
+  for (int v : {rc(0, 2, 1, 0, 0), rc(0, 1, 1, 0, 0), rc(0, 0, 1, 0, 0), rc(1, 1, 1, 0, 0), rc(1, 0, 1, 0, 0),
+                rc(2, 2, 1, 0, 0), rc(2, 0, 1, 0, 0), rc(0, 0, 0, 1, 0)})
+    std::printf(" %d", v);
+}
+""")
+    pkg = os.path.join(ROOT, "deepseek-v4-flash-offload_amd")
+    so = os.path.join(pkg, "dsv4_hip", "libdsv4hip.so")
+    exe = tmp_path / "t"
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-w", "-I/opt/rocm/include",
+                    "-I" + os.path.join(pkg, "csrc"), str(src), so, "-L/opt/rocm/lib", "-lamdhip64",
+                    "-Wl,-rpath,/opt/rocm/lib:" + os.path.dirname(so), "-o", str(exe)], check=True)
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, env=env, timeout=120).stdout.split()
+    assert out[1:] == [out[0]] * 8, out
 
 
 def test_ops_reject_cpu_tensors():
