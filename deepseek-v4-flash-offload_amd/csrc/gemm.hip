@@ -581,8 +581,12 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
 // The weight layout is chosen per block, before anything else, so the two
 // bodies share no live values (a branch around the inner loop alone raised
 // the register count by up to 100 VGPRs).
+// Three waves per SIMD for the bf16 form at K = 512, whose registers lie at the edge (168 of 512
+// per wave): with the weights as the MFMA's first operand the down GEMM took 172 and two waves,
+// 12.6 us for 64 rows and 53.8 for 1024 over 256 experts (D 4096); with the bound 154 and 11.4,
+// 50.5; with the operands the other way 164 and 11.6, 51.4.
 template <int AFMT, bool GATEUP, int NST, bool SH>
-__global__ __launch_bounds__(64 * kWaves) void moe_gemm_kernel(Dsv4GemmArgs p) {
+__global__ __launch_bounds__(64 * kWaves, AFMT == kAfmtBf16 && NST == 2 ? 3 : 1) void moe_gemm_kernel(Dsv4GemmArgs p) {
   // The shared expert's blocks lead the layout and run as two workgroups per 32 (gate/up) or
   // 64 (down) columns: its E4M3 rows are twice as long as a routed expert's, and one
   // workgroup that took the tiles in two passes over K was the launch's tail at small
