@@ -456,6 +456,18 @@ static int hot_rows_threshold(int64_t R, bool pure) {
 // from there on, where the Zipf-hot experts receive hundreds of rows.
 static int layer_block_m(int64_t R) { return R >= 2048 ? 64 : DSV4_GEMM_BLOCK_M; }
 
+// Blocks of the fused shared expert that the 16-row kernel runs as two workgroups each: all
+// of them where there is one (up to 16 tokens), or where the routed experts' gate/up
+// workgroups do not fill the chip's 1024 SIMDs twice; else none. Layer us split / not, top-8:
+// 256 experts, hidden 4096, inter 2048: 1 token 51.1 / 60.5, 8 145.4 / 146.0, 16 223.7 /
+// 224.5, 24 268.9 / 268.1, 32 315.0 / 313.6, 64 434.6 / 426.0, 128 559.4 / 554.6; 128
+// experts, 4096, 1024: 64 tokens 161.1 / 160.2; 64 experts, 2048, 1024: 64 tokens 69.0 / 69.3,
+// 200 109.8 / 110.3; 32 experts, 1024, 512: 64 tokens 35.9 / 38.1, 200 47.2 / 47.1.
+static int shared_split(int T, int R, int E, int I) {
+  const int blocks = (T + DSV4_GEMM_BLOCK_M - 1) / DSV4_GEMM_BLOCK_M;
+  return blocks == 1 || (int64_t)std::min(E, R) * (I / 32) <= 2048 ? blocks : 0;
+}
+
 static LayerWs layer_ws(int T, int K, int E, int D, int I, int profile, bool shared = false,
                         bool routed = false) {
   LayerWs w{};
@@ -691,7 +703,7 @@ static int layer_forward(int profile, int scale_rule, const void* x, const void*
   }
   if (shared) {  // rows R.. read x row f - R with routing weight 1
     gu.has_shared = 1;
-    gu.shared_blocks = (n_sh + bm - 1) / bm;
+    gu.shared_split = shared_split(T, R, E, I);
     gu.shared_expert = E;
     gu.shared_a_rows = n_sh;
     gu.shared = *shared;
@@ -771,7 +783,7 @@ static int layer_forward(int profile, int scale_rule, const void* x, const void*
   dn.out = (uint16_t*)(base + w.out);
   if (shared) {  // h rows are indexed by flat index for every group
     dn.has_shared = 1;
-    dn.shared_blocks = (n_sh + bm - 1) / bm;
+    dn.shared_split = gu.shared_split;
     dn.shared_expert = E;
     dn.shared = *shared;
   }

@@ -100,8 +100,8 @@ struct AStage<kAfmtBf16> {
 // B operand of one stage: E2M1 weights (16 bytes per lane per MFMA, kNT tiles)
 // or, for the shared expert, E4M3 weights (32 bytes, laid out like the E4M3 A
 // operand). An E4M3 stage holds kNT/2 tiles, so both take the same registers;
-// the 64-row kernel covers its kNT tiles in two passes over K and the 16-row one gives
-// them to two workgroups.
+// the E4M3 path covers its kNT tiles in two passes over K (the 16-row kernel by two
+// workgroups where that is faster).
 template <bool B8>
 struct BStageT {
   static constexpr int NTB = B8 ? kNT / 2 : kNT;
@@ -431,6 +431,7 @@ DSV4_DEV void quantise_h_mxfp4(const Dsv4GemmArgs& p, const uint32_t (*hb)[2], i
   if (g == 0) p.hq_scale[(int64_t)f * (p.N / 32) + col0 / 32] = (uint8_t)(k + 127);
 }
 
+// SH: a block of the shared expert, half of whose columns this call takes (`half`).
 // NTW: the block's routed weights are MFMA-tiled and loaded non-temporally.
 template <int AFMT, bool GATEUP, int NST, bool SH, bool NTW>
 __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& p, const int mb, const int e, const int half) {
@@ -442,9 +443,7 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
   // against 15.2 us at one token, 57.4 in both at 8. The down GEMM (188 -> 187 us at 203
   // tokens) and the gate/up that quantises whole 32-column blocks of h (332 -> 330) take it.
   constexpr bool kWRows = !GATEUP || AFMT == 1;
-  // the shared expert's blocks carry id shared_expert and read its E4M3 weights
-  const bool shared = SH && e == p.shared_expert;
-  const Dsv4ExpertPtrs ex = shared ? p.shared : p.experts[e];
+  const Dsv4ExpertPtrs ex = SH ? p.shared : p.experts[e];
   // an expert whose weights are not in the table contributes zeros (never read null)
   const bool have_w = GATEUP ? (ex.w1p && ex.w1s && ex.w3p && ex.w3s) : (ex.w2p && ex.w2s);
   const int r16 = lane & 15, g = lane >> 4;
@@ -455,14 +454,14 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
   const uint8_t* asbase = AFMT == kAfmtBf16 ? nullptr : p.a_scale + arow * (int64_t)(p.Kdim / 32);
 
   // weight rows of this lane's tiles (E2M1: K/2 bytes per row, E4M3: K)
-  const int64_t brow_bytes = shared ? p.Kdim : p.Kdim / 2, bsrow = p.Kdim / 32;
+  const int64_t brow_bytes = SH ? p.Kdim : p.Kdim / 2, bsrow = p.Kdim / 32;
   int col0;
   const uint8_t* bt[kNT];
   const uint8_t* bst[kNT];
   BLayout lay{128, 16};  // routed E2M1 weights: checkpoint or MFMA-tiled layout (table pointer bit 0)
   if (GATEUP) {
     col0 = blockIdx.x * (kWaves * 32) + wave * 32;  // 32 intermediate columns: 2 gate + 2 up tiles
-    if (shared) {  // E4M3 rows, twice the bytes: 16 columns per workgroup, one gate and one up tile
+    if (SH) {  // E4M3 rows, twice the bytes: 16 columns at a time, one gate and one up tile
       col0 += 16 * half;
       const int64_t row = col0 + r16;
       bt[0] = ex.w1p + row * brow_bytes;
@@ -481,7 +480,7 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
     }
   } else {
     col0 = blockIdx.x * (kWaves * 64) + wave * 64;
-    if (shared) {  // two tiles per workgroup
+    if (SH) {  // two tiles at a time
       col0 += 32 * half;
 #pragma unroll
       for (int t = 0; t < kNT / 2; ++t) {
@@ -552,15 +551,10 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
   if constexpr (NTW) asm volatile("" : "+s"(lay.stage_stride), "+s"(lay.mfma_stride));
   auto routed = [&] { kloop(std::false_type{}, std::integral_constant<bool, NTW>{}); };
   if (have_w) {
-    if constexpr (AFMT == 0 && SH) {  // E4M3 weights only meet E4M3 activations (bf16 profile)
-      if (shared) {
-        kloop(std::true_type{}, std::false_type{});
-      } else {
-        routed();
-      }
-    } else {
+    if constexpr (AFMT == 0 && SH)  // E4M3 weights only meet E4M3 activations (bf16 profile)
+      kloop(std::true_type{}, std::false_type{});
+    else
       routed();
-    }
   }
 
   if (GATEUP && kWRows && p.hq_mode == 2) {  // MXFP4 h: this wave holds whole 32-column blocks
@@ -569,10 +563,9 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
     store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, hb, &f);
     quantise_h_mxfp4(p, hb, f, col0, g);
   } else if constexpr (kWRows) {
-    store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, nullptr, nullptr, shared ? kNT / 2 : kNT);
+    store_tile<GATEUP, SH>(p, acc, mb * kBM, col0, g, r16, nullptr, nullptr, SH ? kNT / 2 : kNT);
   } else {
-    if (shared) store_tile_columns<SH, 1>(p, acc, mb * kBM, col0, g, r16);
-    else store_tile_columns<SH, 2>(p, acc, mb * kBM, col0, g, r16);
+    store_tile_columns<SH, SH ? 1 : 2>(p, acc, mb * kBM, col0, g, r16);
   }
 }
 
@@ -587,22 +580,29 @@ __attribute__((always_inline)) DSV4_DEV void moe_gemm_block(const Dsv4GemmArgs& 
 // 50.5; with the operands the other way 164 and 11.6, 51.4.
 template <int AFMT, bool GATEUP, int NST, bool SH>
 __global__ __launch_bounds__(64 * kWaves, AFMT == kAfmtBf16 && NST == 2 ? 3 : 1) void moe_gemm_kernel(Dsv4GemmArgs p) {
-  // The shared expert's blocks lead the layout and run as two workgroups per 32 (gate/up) or
-  // 64 (down) columns: its E4M3 rows are twice as long as a routed expert's, and one
-  // workgroup that took the tiles in two passes over K was the launch's tail at small
-  // batches (one token, top-6: gate/up 18.0 -> 14.4 us, down 10.9 -> 8.9).
+  // The shared expert's blocks lead the layout. Its E4M3 rows are twice as long as a routed
+  // expert's, so a block's 32 (gate/up) or 64 (down) columns take two passes over K: by two
+  // workgroups (shared_split) where one would be the launch's tail (one token, top-6: gate/up
+  // 18.0 -> 14.4 us, down 10.9 -> 8.9), else by one after the other.
   int mb = blockIdx.y, half = 0;
-  if (SH) {
-    if (mb < 2 * p.shared_blocks) half = mb & 1, mb >>= 1;
-    else mb -= p.shared_blocks;
+  if (SH && p.shared_split) {
+    if (mb < 2 * p.shared_split) half = mb & 1, mb >>= 1;
+    else mb -= p.shared_split;
   }
   if (mb * kBM >= p.num_post_padded[0]) return;
   const int e = p.block_expert[mb];
-  const bool shared = SH && e == p.shared_expert;
-  if (kNtLoads && !shared && tiled_ptr(GATEUP ? p.experts[e].w1p : p.experts[e].w2p))
-    moe_gemm_block<AFMT, GATEUP, NST, SH, true>(p, mb, e, half);
+  if constexpr (SH) {  // blocks with id shared_expert; a body of its own: 16 registers fewer in the down GEMM
+    if (e == p.shared_expert) {
+      const int last = p.shared_split ? half : 1;
+#pragma unroll 1
+      for (; half <= last; ++half) moe_gemm_block<AFMT, GATEUP, NST, true, false>(p, mb, e, half);
+      return;
+    }
+  }
+  if (kNtLoads && tiled_ptr(GATEUP ? p.experts[e].w1p : p.experts[e].w2p))
+    moe_gemm_block<AFMT, GATEUP, NST, false, true>(p, mb, e, 0);
   else
-    moe_gemm_block<AFMT, GATEUP, NST, SH, false>(p, mb, e, half);
+    moe_gemm_block<AFMT, GATEUP, NST, false, false>(p, mb, e, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1040,7 +1040,7 @@ template <bool GATEUP, int NST, bool SH>
 static void launch_nst_sh(const Dsv4GemmArgs& a, hipStream_t st) {
   const int cols_per_wave = GATEUP ? 32 : 64;
   if (a.block_m == kBM) {  // decode-shaped: single-wave workgroups
-    const dim3 grid(a.N / (kWaves * cols_per_wave), a.max_blocks + (SH ? a.shared_blocks : 0));
+    const dim3 grid(a.N / (kWaves * cols_per_wave), a.max_blocks + (SH ? a.shared_split : 0));
     if constexpr (!SH) {  // bf16 activations: routed experts only
       if (a.afmt == kAfmtBf16) {
         hipLaunchKernelGGL((moe_gemm_kernel<kAfmtBf16, GATEUP, NST, false>), grid, dim3(64 * kWaves), 0, st, a);
@@ -1099,10 +1099,9 @@ static hipError_t launch(const Dsv4GemmArgs& a, hipStream_t st) {
   // bf16 activations: 16- or 64-row blocks, without a shared expert or a fused h quantisation
   if (a.afmt == kAfmtBf16 && (a.block_m == 128 || a.has_shared || (GATEUP && a.hq_mode))) return hipErrorInvalidValue;
   // the 16-row gate/up quantises h only to MXFP4 and only with E2M1 activations (a wave holds no
-  // whole FP8 block; the E4M3 and bf16 forms always write h), and needs the shared blocks' count
+  // whole FP8 block; the E4M3 and bf16 forms always write h)
   if (a.block_m == kBM && GATEUP && (a.hq_mode || a.hq_skip_h) && !(a.afmt == 1 && a.hq_mode == 2))
     return hipErrorInvalidValue;
-  if (a.block_m == kBM && a.has_shared && a.shared_blocks <= 0) return hipErrorInvalidValue;
   switch (a.Kdim / kStageK) {
     case 2: launch_nst<GATEUP, 2>(a, st); break;
     case 4: launch_nst<GATEUP, 4>(a, st); break;

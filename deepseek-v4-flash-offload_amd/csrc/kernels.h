@@ -145,9 +145,10 @@ struct Dsv4GemmArgs {
   //   w1/w3 [N, K] / w2 [D, I] with E8M0 per 32 along K ([N, K/32], the 128x128
   //   block scales repeated). The last shared_a_rows flat indices below R are
   //   shared-expert rows: A row f - (R - shared_a_rows), routing weight 1.
-  //   shared_blocks: how many blocks it has, the first of the layout (16-row kernel only).
+  //   shared_split (16-row kernel only): how many blocks it has, the first of the layout,
+  //   where each runs as two workgroups; 0: one workgroup each.
   int has_shared;
-  int shared_blocks;
+  int shared_split;
   int shared_expert;
   int shared_a_rows;
   Dsv4ExpertPtrs shared;

@@ -135,22 +135,21 @@ def test_gemm_and_layer_validation():
 def test_gemm_launch_refuses_options_its_kernel_lacks(tmp_path):
     """The internal launchers answer hipErrorInvalidValue, before any launch, for epilogue options the
     16-row gate/up does not have: h quantisation (or leaving h out) with E4M3 or bf16 activations,
-    FP8 h at all, and shared-expert rows without the number of their blocks."""
+    and FP8 h at all."""
     src = tmp_path / "t.cpp"
     src.write_text(r"""
 #include <cstdio>
 #include <initializer_list>
 #include "kernels.h"
 int main() {
-  auto rc = [](int afmt, int hq_mode, int skip, int shared, int shared_blocks) {
+  auto rc = [](int afmt, int hq_mode, int skip) {
     Dsv4GemmArgs g{};
     g.afmt = afmt, g.block_m = 16, g.max_blocks = 1, g.R = 16, g.Kdim = 512, g.N = 512, g.a_row_div = 1;
-    g.hq_mode = hq_mode, g.hq_skip_h = skip, g.has_shared = shared, g.shared_blocks = shared_blocks;
+    g.hq_mode = hq_mode, g.hq_skip_h = skip;
     return (int)launch_moe_gemm_gateup(g, nullptr);
   };
   std::printf("%d", (int)hipErrorInvalidValue);
-  for (int v : {rc(0, 2, 1, 0, 0), rc(0, 1, 1, 0, 0), rc(0, 0, 1, 0, 0), rc(1, 1, 1, 0, 0), rc(1, 0, 1, 0, 0),
-                rc(2, 2, 1, 0, 0), rc(2, 0, 1, 0, 0), rc(0, 0, 0, 1, 0)})
+  for (int v : {rc(0, 2, 1), rc(0, 1, 1), rc(0, 0, 1), rc(1, 1, 1), rc(1, 0, 1), rc(2, 2, 1), rc(2, 0, 1)})
     std::printf(" %d", v);
 }
 """)
@@ -162,7 +161,7 @@ int main() {
                     "-Wl,-rpath,/opt/rocm/lib:" + os.path.dirname(so), "-o", str(exe)], check=True)
     env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, env=env, timeout=120).stdout.split()
-    assert out[1:] == [out[0]] * 8, out
+    assert out[1:] == [out[0]] * 7, out
 
 
 def test_ops_reject_cpu_tensors():

@@ -50,9 +50,11 @@ def test_expand_block_scales_bit_exact(gpu, n, k):
 
 # (T, K, E, D, I): decode at full size, small shapes, 2048 routed rows (64-row
 # blocks, tiled kernel, h quantised in its epilogue), one token, 2400 routed
-# rows (chunked align with the shared group)
+# rows (chunked align with the shared group); the 16-row kernel's shared blocks as
+# one workgroup each (17 and 61 tokens over many experts; the smaller sizes take two)
 CASES = [(8, 8, 256, 4096, 2048), (24, 4, 16, 1024, 512), (256, 8, 16, 1024, 512),
-         (300, 6, 24, 2048, 1024), (1, 8, 64, 1024, 512), (300, 8, 64, 1024, 512)]
+         (300, 6, 24, 2048, 1024), (1, 8, 64, 1024, 512), (300, 8, 64, 1024, 512),
+         (17, 8, 64, 1024, 2048), (61, 4, 128, 1024, 1024)]
 
 
 @pytest.mark.parametrize("T,K,E,D,I", CASES)
