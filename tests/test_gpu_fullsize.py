@@ -7,9 +7,11 @@ against the oracle run on a few of its tokens. Sizes: 256 experts, top-8,
 hidden 4096, inter 2048, at
 * 2048 tokens in both profiles: 16,384 routed rows, 64-row blocks, the chunked
   align, Zipf-hot experts spread over dozens of blocks;
-* 16384 tokens in both profiles: 131,072 routed rows; experts with at least 256
-  rows (the Zipf-hot ones, up to ~14,000 rows) run in 256-row blocks on the
-  large-tile kernel, the others in 64-row blocks;
+  (experts with at least 128 rows in 256-row blocks on the large-tile kernel);
+* 4096 tokens (the same) and 16384 tokens in both profiles: at 131,072 routed
+  rows the experts with at least 64 rows (up to ~14,000) run on the large-tile
+  kernel, whose workgroups take 128-row halves of the 256-row blocks, the others
+  in 64-row blocks;
 * 64 tokens in the a4w4 profile: 512 routed rows on the 16-row kernel;
 * 2048 and 16384 tokens in the pure-bf16 variant (no FP8 round trips): bf16
   activations in 64-row blocks on the tiled kernel; at 16384 tokens (from
@@ -19,8 +21,10 @@ Expert weights are random bytes generated on the device and stored MFMA-tiled,
 as the slot cache stores them. The oracle reads checkpoint-layout copies of the
 sampled tokens' experts. The sample at 2048 tokens: the tokens of the first and
 last routed row of every M block of the 16 hottest experts (the block edges of
-every hot expert; ~260 tokens) plus 32 random ones; at 16384 tokens the same for
-the 8 hottest experts in their 256-row blocks; at 64 tokens, all of them.
+every hot expert; ~260 tokens) plus 32 random ones; where the layer splits the
+same for the 8 hottest experts in their 128-row halves (pure bf16: 256-row
+blocks), and up to 4 experts each with 56-63, 64-127 and 129-191 rows; at 64
+tokens, all of them.
 Tolerances: max relative error (normwise) 1e-2 for bf16 and pure bf16, 2e-2 for
 a4w4; per element, bf16 within 3e-2 and pure bf16 within 2e-2 of
 max(|ref|, rms(ref)), a4w4 bit for bit."""
@@ -102,30 +106,28 @@ def _sample_tokens(ids, T, profile, n_hot=16, n_random=32):
     """Tokens of the first and last routed row of every M block of the n_hot
     hottest experts (rows of an expert in flat-index order, blocks of the
     layer's block size: 64 rows from 2048 routed rows on, else 16), plus
-    n_random random tokens; every token when T <= 64. The large-tile split
-    (from 16,384 routed rows; only the 8 hottest experts are then taken)
-    gives its experts blocks of the rows one workgroup takes: bf16, experts
-    with at least 128 rows, 128 rows (half a hot block); pure bf16 (from
-    65,536 routed rows), experts with at least 128 rows in whole 256-row
-    blocks; a4w4, experts with at
-    least 128 rows in 128-row halves below 32,768 routed rows, then at least
-    256 rows (128 from 65,536) in whole 256-row blocks."""
+    n_random random tokens; every token when T <= 64. In a layer with the
+    large-tile split (from 16,384 routed rows, pure bf16 from 65,536; only the
+    8 hottest experts are then taken) an expert with at least 128 rows, or from
+    40,000 routed rows 64 (pure bf16: 128), has the rows one workgroup takes in
+    place of a block: 128, half of a 256-row block (pure bf16: all of it). Up to
+    4 experts each with 56-63, 64-127 and 129-191 rows are then taken too."""
     if T <= 64:
         return np.arange(T)
     R = ids.size
     flat = ids.reshape(-1)
     counts = np.bincount(flat, minlength=E)
     picks = set()
-    fp8 = profile == "bf16"
     pure = profile == "bf16_pure"
     split = R >= (65536 if pure else 16384)  # the layer's large-tile split
-    hot_min = 128 if (fp8 or pure or R < 32768 or R >= 65536) else 256
+    hot_min = 64 if not pure and R >= 40000 else 128
+    take = list(np.argsort(-counts, kind="stable")[:8 if split else n_hot])
     if split:
-        n_hot = 8
-    for e in np.argsort(-counts, kind="stable")[:n_hot]:
+        for lo, hi in ((56, 63), (64, 127), (129, 191)):
+            take += list(np.nonzero((counts >= lo) & (counts <= hi))[0][:4])
+    for e in take:
         tok = np.nonzero(flat == e)[0] // ids.shape[1]
-        big = 256 if pure else 128 if (fp8 or R < 32768) else 256
-        bm = big if (split and tok.size >= hot_min) else (64 if R >= 2048 else 16)
+        bm = (256 if pure else 128) if (split and tok.size >= hot_min) else (64 if R >= 2048 else 16)
         for b in range(0, tok.size, bm):
             picks.add(int(tok[b]))
             picks.add(int(tok[min(b + bm, tok.size) - 1]))

@@ -57,8 +57,25 @@ def make_layer(E, D, I, experts_needed, dev):
     return host, devw, ops.expert_table(devw, E, dev)
 
 
-def _case(T, K, E, D, I, seed, dev):
-    ids = synth.zipf_topk(T, K, E, synth.rank_permutation(E, 3), np.random.default_rng(seed))
+# rows of an expert around the edges of 64-row blocks, of the large tile's 128-row halves and their
+# 32-row wave tiles, of 256-row blocks and of the layer's 64- and 128-row thresholds
+EDGE_COUNTS = (1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320)
+
+
+def _edge_ids(T, K, seed):
+    """ids [T, K] over 16 experts: expert 1 + i has exactly EDGE_COUNTS[i] rows, expert 0 the others."""
+    flat = np.zeros(T * K, np.int64)
+    at = np.random.default_rng(seed).permutation(T * K)
+    o = 0
+    for i, c in enumerate(EDGE_COUNTS):
+        flat[at[o:o + c]] = i + 1
+        o += c
+    return flat.reshape(T, K)
+
+
+def _case(T, K, E, D, I, seed, dev, ids=None):
+    if ids is None:
+        ids = synth.zipf_topk(T, K, E, synth.rank_permutation(E, 3), np.random.default_rng(seed))
     w = synth.routing_weights(T, K, seed + 1)
     x = synth.bf16_normal(np.random.default_rng(seed + 2), (T, D))
     xb = x.view(torch.int16).numpy().view(np.uint16)
@@ -74,20 +91,26 @@ def _case(T, K, E, D, I, seed, dev):
                                           (640, 8, 8, 4096, 2048, 256)])
 def test_grouped_gemm_stages(gpu, profile, T, K, E, D, I, bm):
     # bm 16 runs the single-wave decode kernel, 64/128 the LDS-tiled kernel, 256 the
-    # large-tile kernel (256 x 256 workgroup tiles, 32x32x64 MFMA) in half-block
-    # workgroups (E4M3 always, E2M1 below 32,768 routed rows)
+    # large-tile kernel (32x32x64 MFMA) in workgroups of half a block each
     _stage_case(gpu, profile, T, K, E, D, I, bm)
 
 
-def test_grouped_gemm_stages_whole_blocks_a4w4(gpu):
-    # from 32,768 routed rows the E2M1 large-tile kernel runs one 8-wave workgroup
-    # per whole 256-row block (csrc/gemm_big.hip launch_moe_gemm_big); every element
-    # of both stages against the oracle, the down GEMM bit for bit
+@pytest.mark.parametrize("profile", ["bf16", "a4w4"])
+@pytest.mark.parametrize("bm", [16, 64, 128, 256])
+def test_grouped_gemm_stages_row_counts(gpu, profile, bm):
+    # every element of both stages, the a4w4 down GEMM bit for bit; with 256-row blocks the
+    # counts leave second halves without a row (they exit) and waves without one (loads and
+    # barriers only)
+    _stage_case(gpu, profile, 600, 4, 16, 1024, 1024, bm, _edge_ids(600, 4, bm))
+
+
+def test_grouped_gemm_stages_many_blocks_a4w4(gpu):
+    # 32,768 routed rows: more large-tile workgroups than the CUs hold at once
     _stage_case(gpu, "a4w4", 4096, 8, 16, 1024, 1024, 256)
 
 
-def _stage_case(gpu, profile, T, K, E, D, I, bm):
-    ids, w, xb, host, devw, table = _case(T, K, E, D, I, 31 + T, gpu)
+def _stage_case(gpu, profile, T, K, E, D, I, bm, ids=None):
+    ids, w, xb, host, devw, table = _case(T, K, E, D, I, 31 + T, gpu, ids)
     al = ops.moe_align(_dev(ids, gpu), _dev(w, gpu), E, bm)
     R = T * K
     if profile == "bf16":
@@ -311,6 +334,66 @@ def test_layer_forward_vs_oracle(gpu, profile, T, K, E, D, I):
         assert np.array_equal(_bits(y), ref["y"])
 
 
+def _largest_products(ref, host, n):
+    """[n, D]: for each output of the oracle's layer, the sum over the token's rows of max_j |h_j w2_j|."""
+    al = ref["align"]
+    h = np.abs(Q.bf16_bits_to_f32(ref["hq"]))
+    out = np.zeros((n, next(iter(host.values()))["w2p"].shape[0]))
+    w2 = {}
+    for r, (e, tok) in enumerate(zip(al["s_e"], al["row"])):
+        if e not in w2:
+            w2[e] = np.abs(Q.dequant_fp4_weight_f32(host[e]["w2p"], host[e]["w2s"]))
+        out[tok] += (w2[e] * h[r]).max(1)
+    return out
+
+
+# the routed rows from which the layer splits, takes 64-row experts too, and (pure bf16) splits, and one fewer
+@pytest.mark.parametrize("profile,T,K", [("bf16", 5461, 3), ("bf16", 2048, 8), ("bf16", 13333, 3), ("bf16", 5000, 8),
+                                         ("a4w4", 5461, 3), ("a4w4", 2048, 8), ("a4w4", 13333, 3), ("a4w4", 5000, 8),
+                                         ("bf16_pure", 21845, 3), ("bf16_pure", 8192, 8)])
+def test_layer_split_edges_vs_oracle(gpu, profile, T, K):
+    """Experts with row counts around the thresholds and block edges, h quantised in every kernel's
+    epilogue: the tokens of each such expert's first and last rows, of the rows around its 32-row
+    tiles, and of 32 rows of expert 0."""
+    E, D, I = 16, 1024, 1024
+    ids, w, xb, host, devw, table = _case(T, K, E, D, I, 91 + T, gpu, _edge_ids(T, K, T))
+    prof = {"bf16": PROFILE_BF16, "a4w4": PROFILE_A4W4, "bf16_pure": PROFILE_BF16_PURE}[profile]
+    y = ops.LayerRunner(gpu, E, D, I).forward(_dev_bf16(xb, gpu), _dev(ids, gpu), _dev(w, gpu), table, profile=prof,
+                                              rule=RULE_OCP_FLOOR)
+    torch.cuda.synchronize()
+    picks = set()
+    for e in range(E):
+        tok = np.nonzero(ids.reshape(-1) == e)[0] // K
+        if e == 0:
+            picks.update(tok[:16].tolist() + tok[-16:].tolist())
+            continue
+        edges = np.arange(0, tok.size, 32)
+        picks.update(tok[edges].tolist() + tok[edges - 1].tolist())  # (edge 0 - 1: the last row)
+    t = np.array(sorted(picks))
+    if profile == "a4w4":
+        ref = M.routed_a4w4(xb[t], ids[t], w[t], host, n_experts=E, rule="ocp_floor", workers=16)
+    else:
+        ref = M.routed_bf16(xb[t], ids[t], w[t], host, n_experts=E, fp8_act=profile == "bf16", workers=16)
+    got, want = Q.bf16_bits_to_f32(_bits(y)), Q.bf16_bits_to_f32(ref["y"])
+    assert np.isfinite(got).all()
+    er = elementwise_rel(got[t], want)
+    print(f"split edges {profile} T={T} K={K}: {t.size} tokens, normwise rel {rel(got[t], want):.3e}, "
+          f"elementwise rel {er:.3e}", flush=True)
+    assert rel(got[t], want) <= TOL[profile]
+    if profile == "bf16":
+        # A bf16 ulp of a gate or up sum may move an E4M3 code of h by one step, at most 2^-3 of its
+        # value. With three rows to a token instead of eight one such step in an output's largest
+        # product can exceed the 3e-2: it may be off by such a step in each of the token's rows instead.
+        step = _largest_products(ref, host, t.size) * 2.0 ** -3
+        err, size = np.abs(got[t].astype(np.float64) - want), np.abs(want.astype(np.float64))
+        floor = np.maximum(size, np.sqrt((size * size).mean()))
+        assert (err <= np.maximum(ELEM_TOL[profile] * floor, step)).all()
+    else:
+        assert er <= ELEM_TOL[profile]
+    if profile == "a4w4":
+        assert np.array_equal(_bits(y)[t], ref["y"])
+
+
 def test_layer_forward_ceil_rule_and_int32_ids(gpu):
     T, K, E, D, I = 16, 4, 16, 512, 512
     ids, w, xb, host, devw, table = _case(T, K, E, D, I, 5, gpu)
@@ -343,8 +426,16 @@ def test_grouped_gemm_stages_bf16_pure(gpu, T, K, E, D, I, block_m):
     # 4-wave gate/up, and no down, whose reduction length must be a multiple of 256); 256-row
     # blocks: the large-tile bf16 kernel (32x32x16 bf16 MFMAs, weight fragments
     # dequantised in registers per 16-k chunk; hidden and inter multiples of 1024)
-    from dsv4_hip import AFMT_BF16
-    ids, w, xb, host, devw, table = _case(T, K, E, D, I, 71 + T, gpu)
+    _pure_stage_case(gpu, T, K, E, D, I, block_m)
+
+
+@pytest.mark.parametrize("block_m", [16, 64, 256])
+def test_grouped_gemm_stages_bf16_pure_row_counts(gpu, block_m):
+    _pure_stage_case(gpu, 600, 4, 16, 1024, 1024, block_m, _edge_ids(600, 4, block_m))
+
+
+def _pure_stage_case(gpu, T, K, E, D, I, block_m, ids=None):
+    ids, w, xb, host, devw, table = _case(T, K, E, D, I, 71 + T, gpu, ids)
     al = ops.moe_align(_dev(ids, gpu), _dev(w, gpu), E, block_m)
     R = T * K
     x = _dev_bf16(xb, gpu)

@@ -84,9 +84,9 @@ def _check(out_w, out_ids, ref_w, ref_ids, scores, bias, K):
     (8, 4096, 256, 8, "sqrtsoftplus", True, True, "bf16"),     # decode
     (64, 4096, 256, 8, "softmax", True, True, "bf16"),
     (2048, 4096, 256, 8, "sigmoid", False, True, "bf16"),      # prefill: 8-wave groups over 256 experts, x in LDS
-    (512, 2048, 256, 8, "softmax", True, True, "fp32"),        # the same with fp32 x
-    (256, 1024, 96, 6, "sqrtsoftplus", True, True, "bf16"),    # 64x32 tiles per wave, 512-k chunks, loads 3 steps ahead
-    (256, 768, 64, 4, "sigmoid", False, True, "fp32"),         # 64x32 tiles, a 768-k chunk: one step ahead
+    (512, 2048, 256, 8, "softmax", True, True, "fp32"),        # 64x32 tiles per wave, 256-k chunks, fp32 x
+    (256, 1024, 96, 6, "sqrtsoftplus", True, True, "bf16"),    # 64x32 tiles, 256-k chunks
+    (256, 768, 64, 4, "sigmoid", False, True, "fp32"),         # 64x32 tiles, 384-k chunks
     (1, 4096, 256, 6, "sqrtsoftplus", True, True, "fp32"),
     (37, 1024, 48, 5, "softmax", False, True, "fp32"),         # E not a multiple of 64, ragged T
     (300, 2048, 512, 8, "sqrtsoftplus", True, False, "bf16"),
@@ -105,10 +105,22 @@ def test_route_matches_oracle(gpu, T, D, E, K, scoring, use_bias, renorm, xdtype
     _check(out_w.cpu().numpy(), out_ids.cpu().numpy(), ref_w, ref_ids, sc, bias, K)
 
 
-@pytest.mark.parametrize("T,D,xdtype", [(8193, 2048, "bf16"), (8200, 1536, "fp32"), (16400, 1024, "bf16")])
-def test_route_several_k_chunks_per_workgroup(gpu, T, D, xdtype):
-    """Token counts that split K in fewer than D / 512 parts: workgroups walk 2 or 3 chunks."""
-    test_route_matches_oracle(gpu, T, D, 256, 6, "sqrtsoftplus", True, True, xdtype)
+def _chunk_k(T, D, E):
+    """k per part of the router's K split (its workspace holds [parts, T, E] fp32)."""
+    parts = ops._lib.lib().dsv4_moe_route_workspace_bytes(T, D, E) // (4 * T * E)
+    return D // parts
+
+
+# From 256 tokens: 512-k parts take x through the LDS where E is a multiple of 256, or else the tile
+# kernel with its loads three steps ahead; parts of 2 and more times 512 k walk chunks (a multiple of
+# 256 experts); the rest take the tile kernel one step ahead
+@pytest.mark.parametrize("xdtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("T,D,E,part", [(2048, 4096, 256, 512), (2048, 4096, 240, 512), (8193, 2048, 256, 1024),
+                                        (16400, 1024, 256, 1024), (16400, 1536, 256, 1536), (4097, 3072, 512, 1536),
+                                        (16385, 2048, 256, 2048), (8200, 1536, 256, 768)])
+def test_route_k_parts(gpu, T, D, E, part, xdtype):
+    assert _chunk_k(T, D, E) == part
+    test_route_matches_oracle(gpu, T, D, E, 6, "sqrtsoftplus", True, True, xdtype)
 
 
 @pytest.mark.parametrize("tab_dtype", [torch.int32, torch.int64])
