@@ -426,7 +426,14 @@ struct LayerWs {
 //   1209 / 1197 / -, 5000 1270 / 1285 / 1281 / -, 6007 1421 / 1462 / 1458 / 1472, 16384 3042 /
 //   3109 / 3153 / 3253.
 // So 128 rows, and 64 from 40,000 routed rows, where the smaller experts' workgroups no
-// longer lengthen the launch by a round of their own.
+// longer lengthen the launch by a round of their own. Where that point lies depends on the
+// number of experts and of N tiles; at other shapes, with 64 / 128 rows (bf16; a4w4):
+//   128 experts, 2048 x 1024: 4500 tokens 387 / 395; 354 / 363, 5120 423 / 441; 384 / 403,
+//   8192 605 / 603; 539 / 540. 64 experts, 4096 x 1024: 5120 tokens 668 / 668; 595 / 595.
+//   256 experts, 2048 x 1024: 4500 tokens 448 / 431; 425 / 402, 5120 485 / 476; 454 / 442,
+//   8192 657 / 677; 602 / 613. 256 experts, 1024 x 1024: 5120 tokens 323 / 312; 305 / 300.
+//   512 experts, uniform: 2048 x 1024, 5120 tokens 606 / 716; 572 / 638, 4096 x 2048 1924 /
+//   2206; 1796 / 1912.
 //   From 16,384 routed rows: splitting at 600, 1024 and 1500 tokens with 128 (64) rows
 //   gave 653 (652), 734 (721), 777 (771) against 663, 717, 791 without (bf16), 645 (634),
 //   710 (693), 743 (730) against 635, 682, 744 (a4w4).
